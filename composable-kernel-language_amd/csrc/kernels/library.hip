@@ -101,14 +101,17 @@ __device__ __forceinline__ int load_position(const int *position) { return *posi
 // reads of a 2 GiB buffer stream at ~7.1 TB/s this way against ~6.1 TB/s with the default
 // policy; but a decode step whose few MB of weights stay in the caches between steps runs
 // slower with it, and a branch between the two in one kernel costs the small launches too.
-typedef float stream_float4 __attribute__((ext_vector_type(4)));
-typedef float stream_float2 __attribute__((ext_vector_type(2)));
+// The vector types are only 4-byte aligned: a global 8- or 16-byte access needs no more on gfx950,
+// so rows of any length (O or I of a linear not a multiple of 4) take the same instructions.
+typedef float stream_float4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float stream_float2 __attribute__((ext_vector_type(2), aligned(4)));
 template <bool NT> __device__ __forceinline__ float4 load4(const float *p) {
   if constexpr (NT) {
     stream_float4 v = __builtin_nontemporal_load(reinterpret_cast<const stream_float4 *>(p));
     return make_float4(v.x, v.y, v.z, v.w);
   } else {
-    return *reinterpret_cast<const float4 *>(p);
+    stream_float4 v = *reinterpret_cast<const stream_float4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
   }
 }
 template <bool NT> __device__ __forceinline__ float2 load2(const float *p) {
@@ -116,7 +119,8 @@ template <bool NT> __device__ __forceinline__ float2 load2(const float *p) {
     stream_float2 v = __builtin_nontemporal_load(reinterpret_cast<const stream_float2 *>(p));
     return make_float2(v.x, v.y);
   } else {
-    return *reinterpret_cast<const float2 *>(p);
+    stream_float2 v = *reinterpret_cast<const stream_float2 *>(p);
+    return make_float2(v.x, v.y);
   }
 }
 template <bool NT> __device__ __forceinline__ float load1(const float *p) {
@@ -606,8 +610,8 @@ template <int J, bool NT> __device__ __forceinline__ void load_columns(float (&o
 }
 
 template <int J> __device__ __forceinline__ void store_columns(float *p, const float (&v)[J]) {
-  if constexpr (J == 4) *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  else if constexpr (J == 2) *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
+  if constexpr (J == 4) *reinterpret_cast<stream_float4 *>(p) = stream_float4{v[0], v[1], v[2], v[3]};
+  else if constexpr (J == 2) *reinterpret_cast<stream_float2 *>(p) = stream_float2{v[0], v[1]};
   else *p = v[0];
 }
 
@@ -633,7 +637,7 @@ __device__ __forceinline__ void mfma_load(MfmaStage<J, S, M> &st, const float *x
   for (int u = 0; u < 2 * S; ++u) {
     const int kk = k + 8 * u;
     if constexpr (!Tail) {
-      float4 v = *reinterpret_cast<const float4 *>(dead ? zero : xr + kk);
+      float4 v = load4<false>(dead ? zero : xr + kk);
       st.x[u][0] = v.x; st.x[u][1] = v.y; st.x[u][2] = v.z; st.x[u][3] = v.w;
     }
 #pragma unroll
@@ -682,8 +686,11 @@ __device__ void linear_mfma(const LinearArgs *a, int block, float *smem) {
   const int m = lane & 31, s = lane >> 5;
   const int tn = block % a0.tilesN, rest = block / a0.tilesN;
   const int kg = rest % a0.kSplit, rt = rest / a0.kSplit;
-  const int n = tn * 32 * J + J * m;               // first of this lane's J columns
-  const bool colOk = n < a0.O;                     // host guarantees O % J == 0
+  // First of this lane's J columns. A lane whose columns would run past O (O % J != 0) takes the
+  // last J columns instead: it computes some of its neighbour's columns again, from the same
+  // products in the same order, so both store the same values.
+  const bool colOk = tn * 32 * J + J * m < a0.O;
+  const int n = min(tn * 32 * J + J * m, a0.O - J);   // host guarantees O >= J
   const int row = rt * 32 + m;
   const bool rowOk = row < a0.B;
   const float *xr = a0.x + long(rowOk ? row : 0) * a0.I;
