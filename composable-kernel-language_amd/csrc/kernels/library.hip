@@ -575,26 +575,68 @@ __device__ __forceinline__ bool split_arrive(unsigned *counter, int parts) {
 }
 
 // Adds the kSplit partial tiles (rows [r0, r0+rows), columns [c0, c0+cols)) in split order
-// and writes dst. The partials of kFinishBatch splits are loaded together, then added in order
-// (the batch condition is uniform; agent-coherent loads of one address serialize, so indices past
-// the end are skipped rather than clamped).
+// and writes dst. What bounds it is the round trip of an agent-coherent load (it goes past the L2
+// of this XCD), so a thread requests the planes of U pairs of columns, kFinishBatch splits of each,
+// before it adds any. Against one column at a time, cold weights, ordinary launches: 32 x 2048 x 2048
+// 13.1 -> 9.8 us, 32 x 2048 x 5632 23.9 -> 17.1 us, 32 x 5632 x 2048 18.3 -> 14.6 us.
+// The batch condition is uniform; agent-coherent loads of one address serialize, so splits past
+// the end are skipped rather than clamped, and a unit past the end repeats the thread's own first
+// one. Pairs need an even row length; other rows go one column at a time.
 constexpr int kFinishBatch = 8;
-__device__ void split_finish(const LinearArgs &a, const float *partial, long planeStride, int r0, int rows, int c0,
-                             int cols) {
-  for (int e = threadIdx.x; e < rows * cols; e += blockDim.x) {
-    int r = r0 + e / cols, c = c0 + e % cols;
-    if (r >= a.B || c >= a.O) continue;
-    const float *p = partial + long(r) * a.O + c;
-    float total = 0.f;
-    for (int g0 = 0; g0 < a.kSplit; g0 += kFinishBatch) {
-      float v[kFinishBatch];
-#pragma unroll
-      for (int j = 0; j < kFinishBatch; ++j) v[j] = g0 + j < a.kSplit ? partial_load(p + (g0 + j) * planeStride) : 0.f;
-#pragma unroll
-      for (int j = 0; j < kFinishBatch; ++j) total += v[j];
-    }
-    a.dst[long(r) * a.O + c] = total;
+template <int N> struct FinishValue { float v[N]; };
+template <int N> __device__ __forceinline__ FinishValue<N> partial_load_n(const float *p) {
+  FinishValue<N> out;
+  if constexpr (N == 2) {
+    const unsigned long long bits = __hip_atomic_load(
+        reinterpret_cast<unsigned long long *>(const_cast<float *>(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    out.v[0] = __uint_as_float(unsigned(bits));
+    out.v[1] = __uint_as_float(unsigned(bits >> 32));
+  } else {
+    out.v[0] = partial_load(p);
   }
+  return out;
+}
+template <int U, int N>
+__device__ __forceinline__ void split_finish_columns(const LinearArgs &a, const float *partial, long planeStride, int r0,
+                                                     int rows, int c0, int cols) {
+  const int per = min(cols, a.O - c0) / N, units = min(rows, a.B - r0) * per, step = blockDim.x;
+  for (int e0 = threadIdx.x; e0 < units; e0 += U * step) {
+    FinishValue<N> total[U];
+    int at[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + u * step < units ? e0 + u * step : e0;
+      at[u] = (r0 + e / per) * a.O + c0 + N * (e % per);
+#pragma unroll
+      for (int k = 0; k < N; ++k) total[u].v[k] = 0.f;
+    }
+    for (int g0 = 0; g0 < a.kSplit; g0 += kFinishBatch) {
+      FinishValue<N> v[kFinishBatch][U];
+#pragma unroll
+      for (int j = 0; j < kFinishBatch; ++j)
+        if (g0 + j < a.kSplit) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[j][u] = partial_load_n<N>(partial + (g0 + j) * planeStride + at[u]);
+        }
+#pragma unroll
+      for (int j = 0; j < kFinishBatch; ++j)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < N; ++k) total[u].v[k] += g0 + j < a.kSplit ? v[j][u].v[k] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if constexpr (N == 2) *reinterpret_cast<stream_float2 *>(a.dst + at[u]) = stream_float2{total[u].v[0], total[u].v[1]};
+      else a.dst[at[u]] = total[u].v[0];
+    }
+  }
+}
+template <int U>
+__device__ __forceinline__ void split_finish(const LinearArgs &a, const float *partial, long planeStride, int r0, int rows,
+                                             int c0, int cols) {
+  if ((a.O & 1) == 0) split_finish_columns<U, 2>(a, partial, planeStride, r0, rows, c0, cols);
+  else split_finish_columns<U, 1>(a, partial, planeStride, r0, rows, c0, cols);
 }
 
 template <int J, bool NT> __device__ __forceinline__ void load_columns(float (&out)[J], const float *p) {
@@ -607,6 +649,21 @@ template <int J, bool NT> __device__ __forceinline__ void load_columns(float (&o
   } else {
     out[0] = load1<NT>(p);
   }
+}
+
+// Agent-coherent store of J columns: 64-bit stores when the row length is even (J columns then start
+// at an even element), half the instructions and write requests of single words.
+template <int J> __device__ __forceinline__ void partial_store_columns(float *p, const float (&v)[J], bool pairs) {
+  if (J > 1 && pairs) {
+#pragma unroll
+    for (int j = 0; j + 1 < J; j += 2)
+      __hip_atomic_store(reinterpret_cast<unsigned long long *>(p + j),
+                         (static_cast<unsigned long long>(__float_as_uint(v[j + 1])) << 32) | __float_as_uint(v[j]),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) partial_store(p + j, v[j]);
 }
 
 template <int J> __device__ __forceinline__ void store_columns(float *p, const float (&v)[J]) {
@@ -678,7 +735,7 @@ __device__ __forceinline__ void mfma_compute(const MfmaStage<J, S, M> &st, float
 
 // `a` holds M member blocks that agree on x, B, I, O, layer and the tiling (M = 1: one linear);
 // the workgroup computes its tile of every member from one stream of x fragments.
-template <int J, int S, int M, bool NT>
+template <int J, int S, int M, bool NT, bool Combine>
 __device__ void linear_mfma(const LinearArgs *a, int block, float *smem) {
   const LinearArgs &a0 = a[0];
   const int lane = threadIdx.x & 63;
@@ -782,30 +839,41 @@ __device__ void linear_mfma(const LinearArgs *a, int block, float *smem) {
           sum[j][0] += o.x; sum[j][1] += o.y; sum[j][2] += o.z; sum[j][3] += o.w;
         }
       }
+      // Keeps the sums ahead of the stores' row test: sunk into it, the 128-bit LDS reads become
+      // single words.
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(sum[j][q]));
+      float *out = ae.kSplit > 1 ? partial + long(kg) * rowTiles * 32 * O : ae.dst;
+      const bool coherent = Combine && ae.kSplit > 1 && !ae.deferred;
+      const int i0 = rt * 32 + 8 * wave + 4 * s;          // row of accumulator register 4*wave
+      float *p = out + long(i0) * O + n;
       if (colOk) {
+        if (coherent) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int i = rt * 32 + 8 * wave + 4 * s + q;   // row of accumulator register 4*wave + q
-          float v[J];
+          for (int q = 0; q < 4; ++q, p += O) {
+            float v[J];
 #pragma unroll
-          for (int j = 0; j < J; ++j) v[j] = sum[j][q];
-          if (ae.kSplit > 1) {
-            float *p = partial + long(kg) * rowTiles * 32 * O + long(i) * O + n;
-            if (ae.deferred) {
-              store_columns<J>(p, v);
-            } else {
+            for (int j = 0; j < J; ++j) v[j] = sum[j][q];
+            if (i0 + q < ae.B) partial_store_columns<J>(p, v, (O & 1) == 0);
+          }
+        } else {
 #pragma unroll
-              for (int j = 0; j < J; ++j) partial_store(p + j, v[j]);
-            }
-          } else if (i < ae.B) {
-            store_columns<J>(ae.dst + long(i) * O + n, v);
+          for (int q = 0; q < 4; ++q, p += O) {
+            float v[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) v[j] = sum[j][q];
+            if (i0 + q < ae.B) store_columns<J>(p, v);
           }
         }
       }
-      if (ae.kSplit > 1 && !ae.deferred) {
-        unsigned *counters = split_counters(ae);
-        if (split_arrive(counters + rt * ae.tilesN + tn, ae.kSplit))
-          split_finish(ae, partial, long(rowTiles) * 32 * O, rt * 32, 32, tn * 32 * J, 32 * J);
+      if constexpr (Combine) {
+        if (ae.kSplit > 1 && !ae.deferred) {
+          unsigned *counters = split_counters(ae);
+          if (split_arrive(counters + rt * ae.tilesN + tn, ae.kSplit))
+            split_finish<J == 1 ? 2 : 4>(ae, partial, long(rowTiles) * 32 * O, rt * 32, 32, tn * 32 * J, 32 * J);
+        }
       }
     }
   }
@@ -887,42 +955,41 @@ template <bool NT> __device__ void linear_rowvec_stream(const LinearArgs &a, int
     else a.dst[long(b) * a.O + col] = v;
   }
   if (a.kSplit > 1 && !a.deferred && split_arrive(split_counters(a) + b * a.tilesN + tn, a.kSplit))
-    split_finish(a, split_partials(a, true), long(a.B) * a.O, b, 1, tn * 64, 64);
+    split_finish<1>(a, split_partials(a, true), long(a.B) * a.O, b, 1, tn * 64, 64);
 }
 
-template <int J, int S, bool NT = false> __device__ void linear_mfma_body(const LinearArgs &a, int block) {
+template <int J, bool NT, bool Combine> __device__ void linear_mfma_body(const LinearArgs &a, int block) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  linear_mfma<J, S, 1, NT>(&a, block, smem);
+  linear_mfma<J, 1, 1, NT, Combine>(&a, block, smem);
 }
 CKL_ENTRY_ATTR(linear_rowvec, LinearArgs, linear_rowvec_stream<false>, 1024, )
 CKL_ENTRY_ATTR(linear_rowvec_nt, LinearArgs, linear_rowvec_stream<true>, 1024, )
-// ckl_linear_mfma<J>x<S>: J weight columns per lane, 16*S reduction rows per stage.
-CKL_ENTRY(linear_mfma1x1, LinearArgs, (linear_mfma_body<1, 1>))
-CKL_ENTRY(linear_mfma1x1_nt, LinearArgs, (linear_mfma_body<1, 1, true>))
-CKL_ENTRY(linear_mfma1x2, LinearArgs, (linear_mfma_body<1, 2>))
-CKL_ENTRY_ATTR(linear_mfma1x4, LinearArgs, (linear_mfma_body<1, 4>), kBlock, CKL_TWO_WAVES)
-CKL_ENTRY(linear_mfma2x1, LinearArgs, (linear_mfma_body<2, 1>))
-CKL_ENTRY(linear_mfma2x1_nt, LinearArgs, (linear_mfma_body<2, 1, true>))
-CKL_ENTRY_ATTR(linear_mfma2x2, LinearArgs, (linear_mfma_body<2, 2>), kBlock, CKL_TWO_WAVES)
-CKL_ENTRY_ATTR(linear_mfma2x4, LinearArgs, (linear_mfma_body<2, 4>), kBlock, CKL_TWO_WAVES)
-CKL_ENTRY_ATTR(linear_mfma4x1, LinearArgs, (linear_mfma_body<4, 1>), kBlock, CKL_TWO_WAVES)
-CKL_ENTRY_ATTR(linear_mfma4x1_nt, LinearArgs, (linear_mfma_body<4, 1, true>), kBlock, CKL_TWO_WAVES)
-CKL_ENTRY_ATTR(linear_mfma4x2, LinearArgs, (linear_mfma_body<4, 2>), kBlock, CKL_TWO_WAVES)
+// ckl_linear_mfma<J>x1: J weight columns per lane, 16 reduction rows per stage. The `_deferred`
+// entries leave a split's planes to their reader and hold no combine: the combine's registers and
+// code cost a launch that never runs it (large decoder step 727 us without, 734 us with it in its
+// projections). The executor takes them for a launch all of whose members are deferred.
+#define CKL_LINEAR_MFMA(J, attributes)                                                                        \
+  CKL_ENTRY_ATTR(linear_mfma##J##x1, LinearArgs, (linear_mfma_body<J, false, true>), kBlock, attributes)      \
+  CKL_ENTRY_ATTR(linear_mfma##J##x1_nt, LinearArgs, (linear_mfma_body<J, true, true>), kBlock, attributes)    \
+  CKL_ENTRY_ATTR(linear_mfma##J##x1_deferred, LinearArgs, (linear_mfma_body<J, false, false>), kBlock, attributes) \
+  CKL_ENTRY_ATTR(linear_mfma##J##x1_nt_deferred, LinearArgs, (linear_mfma_body<J, true, false>), kBlock, attributes)
+CKL_LINEAR_MFMA(1, )
+CKL_LINEAR_MFMA(2, )
+CKL_LINEAR_MFMA(4, CKL_TWO_WAVES)
 // ckl_linear_mfma<J>x1_shared<M>: M linears of one shape and tiling that multiply the same x
 // (their blocks in a Group<LinearArgs>, count == M; grid = one member's grid). Each workgroup
 // computes its tile of every member from one x stream, so the sibling projections of a decoder
 // layer (q, k, v; gate, up) run as one grid of at most one workgroup per CU.
-#define CKL_LINEAR_SHARED(J, M)                                                                       \
-  extern "C" __global__ __launch_bounds__(kBlock) CKL_ONE_WAVE void ckl_linear_mfma##J##x1_shared##M( \
-      const Group<LinearArgs> g) {                                                                    \
-    extern __shared__ __attribute__((aligned(16))) float smem[];                                                                   \
-    linear_mfma<J, 1, M, false>(g.m, blockIdx.x, smem);                             \
-  }                                                                                                   \
-  extern "C" __global__ __launch_bounds__(kBlock) CKL_ONE_WAVE void ckl_linear_mfma##J##x1_nt_shared##M( \
-      const Group<LinearArgs> g) {                                                                    \
-    extern __shared__ __attribute__((aligned(16))) float smem[];                                                                   \
-    linear_mfma<J, 1, M, true>(g.m, blockIdx.x, smem);                              \
+#define CKL_LINEAR_SHARED_ENTRY(name, J, M, NT, Combine)                                              \
+  extern "C" __global__ __launch_bounds__(kBlock) CKL_ONE_WAVE void name(const Group<LinearArgs> g) { \
+    extern __shared__ __attribute__((aligned(16))) float smem[];                                      \
+    linear_mfma<J, 1, M, NT, Combine>(g.m, blockIdx.x, smem);                                         \
   }
+#define CKL_LINEAR_SHARED(J, M)                                                               \
+  CKL_LINEAR_SHARED_ENTRY(ckl_linear_mfma##J##x1_shared##M, J, M, false, true)                \
+  CKL_LINEAR_SHARED_ENTRY(ckl_linear_mfma##J##x1_nt_shared##M, J, M, true, true)              \
+  CKL_LINEAR_SHARED_ENTRY(ckl_linear_mfma##J##x1_deferred_shared##M, J, M, false, false)      \
+  CKL_LINEAR_SHARED_ENTRY(ckl_linear_mfma##J##x1_nt_deferred_shared##M, J, M, true, false)
 CKL_LINEAR_SHARED(1, 2)
 CKL_LINEAR_SHARED(1, 3)
 CKL_LINEAR_SHARED(2, 2)

@@ -933,6 +933,24 @@ bool sharesOperands(const std::vector<const Launch *> &members) {
   return true;
 }
 
+bool deferredEntry(const Launch &l, std::string &entry) {
+  if (l.name.rfind("ckl_linear_mfma", 0) != 0) return false;
+  const size_t shared = l.name.find("_shared");
+  const std::string plain = l.name.substr(0, shared);
+  if (plain.size() >= 6 && plain.compare(plain.size() - 6, 6, "_group") == 0) return false;
+  const size_t members = shared == std::string::npos ? 1 : size_t(l.name[shared + 7] - '0');
+  if (members < 1 || members > size_t(kMaxGroup) || l.arguments.size() < members * sizeof(LinearArgs)) return false;
+  bool streaming = false;
+  for (size_t m = 0; m < members; ++m) {
+    LinearArgs a;
+    std::memcpy(&a, l.arguments.data() + m * sizeof a, sizeof a);
+    if (!a.deferred) return false;
+    streaming |= int64_t(a.I) * a.O * 4 >= kStreamBytes;
+  }
+  entry = plain + (streaming ? "_nt" : "") + "_deferred" + (shared == std::string::npos ? "" : l.name.substr(shared));
+  return true;
+}
+
 std::map<size_t, Launch> deferCombines(const Plan &plan, const std::vector<bool> &temporary, std::vector<Chain> &chains) {
   auto slotAt = [](const Launch &l, size_t offset) -> int64_t {
     for (size_t s = 0; s < l.slotOffsets.size() && s < l.slotResources.size(); ++s)

@@ -558,7 +558,15 @@ std::vector<Unit> Invocation::buildUnits(int mode, uint64_t batch, const Plan &r
   std::vector<Chain> chains = findChains(plan, temporaryResources);
   std::map<size_t, Launch> deferred = deferCombines(plan, temporaryResources, chains);
   units = groupPlan(repeated, chains, deferred, batch);
-  for (Unit &u : units) prepareParams(u.launch, *device);
+  for (Unit &u : units) {
+    std::string entry;
+    if (deferredEntry(u.launch, entry)) {
+      hipFunction_t function = nullptr;
+      if (hipModuleGetFunction(&function, u.launch.module, entry.c_str()) == hipSuccess) u.launch.function = function;
+      else (void)hipGetLastError();
+    }
+    prepareParams(u.launch, *device);
+  }
   return units;
 }
 

@@ -125,6 +125,9 @@ std::map<size_t, Launch> deferCombines(const Plan &plan, const std::vector<bool>
 // Whether sibling launches of one entry point read the same operand the way its _shared<M> entry
 // point requires (linears multiplying the same x with one shape and tiling).
 bool sharesOperands(const std::vector<const Launch *> &members);
+// Whether every member of a linear launch (alone or shared) leaves its split combine to its reader,
+// and then the entry point without a combine that the launch takes (when the code object has it).
+bool deferredEntry(const Launch &launch, std::string &entry);
 // Whether a library launch streams at least kStreamBytes of weights or cache (its <entry>_nt
 // variant reads them with nontemporal loads).
 bool streams(const Launch &launch);
