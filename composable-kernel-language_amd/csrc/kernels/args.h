@@ -93,6 +93,7 @@ struct CKL_ALIGN UpdateArgs { const float *src; float *dst; float bias; int n; }
 
 // Chains (member blocks back to back, in dispatch order).
 struct CKL_ALIGN RmsChainArgs { RmsStatsArgs stats; RmsApplyArgs apply; };
+struct CKL_ALIGN AddChainArgs { BinaryArgs add; PartialSource x, y; };
 struct CKL_ALIGN AddRmsChainArgs { BinaryArgs add; RmsStatsArgs stats; RmsApplyArgs apply; PartialSource x, y; };
 struct CKL_ALIGN EmbeddingRmsChainArgs { EmbeddingArgs embedding; RmsStatsArgs stats; RmsApplyArgs apply; };
 struct CKL_ALIGN SiluMultiplyChainArgs { UnaryArgs silu; BinaryArgs multiply; PartialSource src, y; };

@@ -1734,6 +1734,22 @@ __device__ void silu__multiply_body(const SiluMultiplyChainArgs &a, int block) {
 }
 CKL_ENTRY(silu__multiply, SiluMultiplyChainArgs, silu__multiply_body)
 
+// add alone, either operand a split linear's partial planes (a residual sum that no norm follows):
+// float4 i or element i per thread, the planes of a batch requested before the first sum. The linear
+// then needs no counter and no coherent loads: MLP 32 x 2048 x 5632 64.9 -> 62.6 us.
+__device__ void add_planes_body(const AddChainArgs &a, int block) {
+  const long i = long(block) * kBlock + threadIdx.x;
+  if ((a.add.n & 3) == 0) {
+    if (i >= a.add.n / 4) return;
+    const float4 x = source4(a.x, a.add.x, 4 * i), y = source4(a.y, a.add.y, 4 * i);
+    reinterpret_cast<float4 *>(a.add.dst)[i] =
+        make_float4(binary<0>(x.x, y.x), binary<0>(x.y, y.y), binary<0>(x.z, y.z), binary<0>(x.w, y.w));
+  } else if (i < a.add.n) {
+    a.add.dst[i] = binary<0>(source1(a.x, a.add.x, i), source1(a.y, a.add.y, i));
+  }
+}
+CKL_ENTRY(add_planes, AddChainArgs, add_planes_body)
+
 
 // Row-parallel linear chains. With one column tile (O <= 64) and one slice a rowvec workgroup
 // holds a whole output row, so the row ops after the linear run in the same workgroup: linear ->

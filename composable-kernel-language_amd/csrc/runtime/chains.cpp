@@ -8,7 +8,8 @@
 // attention_values (or the rope part alone, attention_scores -> softmax -> attention_values, or
 // softmax -> attention_values), greedy -> advance, and for row-parallel linears whose workgroups
 // hold whole rows, linear -> add -> rms_stats -> rms_apply and linear, linear -> silu -> multiply
-// (both as one launch for single-wave linears). The plan itself (nodes, edges,
+// (both as one launch for single-wave linears). add alone is a chain of one, so that it can read a
+// split linear's partial planes. The plan itself (nodes, edges,
 // argument blocks) is unchanged; only the inferred lowering contracts a chain into one unit.
 //
 // A chain is taken only when
@@ -160,6 +161,19 @@ const char *addRmsChain(const Members &m, const Internal &internal, Launch &out)
   ranges.push_back(rows(c.add.dst, count, row, true));
   if (!hazardFree(ranges)) return kOverlap;
   rowGeometry(out, c.stats.B);
+  setArguments(out, c);
+  return nullptr;
+}
+
+// add alone, so that it can read a split linear's partial planes.
+const char *addChain(const Members &m, const Internal &, Launch &out) {
+  AddChainArgs c{block<BinaryArgs>(*m[0]), {}, {}};
+  const uint64_t n = uint64_t(std::max(c.add.n, 0));
+  std::vector<Range> ranges{rows(c.add.x, n, 4, false), rows(c.add.y, n, 4, false), rows(c.add.dst, n, 4, true)};
+  if (!n || !hazardFree(ranges)) return kOverlap;
+  out.grid[0] = cdiv(n % 4 == 0 ? n / 4 : n, 256);
+  out.block[0] = 256;
+  out.shared = 0;
   setArguments(out, c);
   return nullptr;
 }
@@ -727,6 +741,8 @@ const std::vector<Rule> &rules() {
        "ckl_linear_rowvec__linear_rowvec__silu__multiply", linearSiluChain, matchLinearSilu},
       {{"ckl_add", "ckl_rms_stats", "ckl_rms_apply"}, "ckl_add__rms_stats__rms_apply", addRmsChain, nullptr,
        {{0, offsetof(BinaryArgs, x), offsetof(AddRmsChainArgs, x)}, {0, offsetof(BinaryArgs, y), offsetof(AddRmsChainArgs, y)}}},
+      {{"ckl_add"}, "ckl_add_planes", addChain, nullptr,
+       {{0, offsetof(BinaryArgs, x), offsetof(AddChainArgs, x)}, {0, offsetof(BinaryArgs, y), offsetof(AddChainArgs, y)}}},
       {{"ckl_embedding", "ckl_rms_stats", "ckl_rms_apply", "ckl_linear_rowvec", "ckl_linear_rowvec", "ckl_linear_rowvec"},
        "ckl_embedding__rms_stats__rms_apply__linear_rowvec__linear_rowvec__linear_rowvec", embeddingRmsLinearsChain,
        matchEmbeddingRmsLinears},
