@@ -50,8 +50,8 @@ struct CKL_ALIGN LinearArgs {
 // reads zero at every launch, never shared): kLinearZeroPage bytes that stay zero (padding loads
 // read them), then the split completion counters (uint32 per output tile, padded to 256 B; reset
 // by the last workgroup of each tile). `partials` (null when kSplit = 1): the partial planes
-// float[kSplit][rows][O], rows = B for the vector path (ckl_linear_rowvec) and 32 * ceil(B / 32)
-// for the MFMA paths, live from the launch until the readers of dst have run.
+// float[kSplit][rows][O], rows = B for the paths of at most 16 rows (ckl_linear_rowvec,
+// ckl_linear_mfma16_*) and 32 * ceil(B / 32) for the 32-row MFMA paths, live from the launch until the readers of dst have run.
 constexpr int kLinearZeroPage = 256;
 // The MFMA linear's epilogue hands the accumulators of EM members through LDS in one pass:
 // 16 KB per member and weight column of a lane (4 waves x 16 registers x 64 lanes x 4 bytes), at

@@ -30,6 +30,9 @@ constexpr int kBlock = 256;
     body(g.m[m], b - g.start[m]);                                                                     \
   }
 #define CKL_ENTRY(name, Args, body) CKL_ENTRY_ATTR(name, Args, body, kBlock, )
+// An entry the executor never groups.
+#define CKL_SINGLE_ENTRY(name, Args, body, threads, attributes)                                      \
+  extern "C" __global__ __launch_bounds__(threads) attributes void ckl_##name(const Args a) { body(a, blockIdx.x); }
 // Streaming kernels that keep several loads in flight per lane trade occupancy for registers.
 #define CKL_TWO_WAVES __attribute__((amdgpu_waves_per_eu(1, 2)))
 #define CKL_ONE_WAVE __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -955,7 +958,9 @@ template <bool NT> __device__ void linear_rowvec_stream(const LinearArgs &a, int
     else a.dst[long(b) * a.O + col] = v;
   }
   if (a.kSplit > 1 && !a.deferred && split_arrive(split_counters(a) + b * a.tilesN + tn, a.kSplit))
-    split_finish<1>(a, split_partials(a, true), long(a.B) * a.O, b, 1, tn * 64, 64);
+    // One column at a time: 64 columns are one a lane, and the paired form's code and registers cost
+    // the unsplit launches of a small decoder 0.25 us each.
+    split_finish_columns<1, 1>(a, split_partials(a, true), long(a.B) * a.O, b, 1, tn * 64, 64);
 }
 
 template <int J, bool NT, bool Combine> __device__ void linear_mfma_body(const LinearArgs &a, int block) {
@@ -971,8 +976,8 @@ CKL_ENTRY_ATTR(linear_rowvec_nt, LinearArgs, linear_rowvec_stream<true>, 1024, )
 #define CKL_LINEAR_MFMA(J, attributes)                                                                        \
   CKL_ENTRY_ATTR(linear_mfma##J##x1, LinearArgs, (linear_mfma_body<J, false, true>), kBlock, attributes)      \
   CKL_ENTRY_ATTR(linear_mfma##J##x1_nt, LinearArgs, (linear_mfma_body<J, true, true>), kBlock, attributes)    \
-  CKL_ENTRY_ATTR(linear_mfma##J##x1_deferred, LinearArgs, (linear_mfma_body<J, false, false>), kBlock, attributes) \
-  CKL_ENTRY_ATTR(linear_mfma##J##x1_nt_deferred, LinearArgs, (linear_mfma_body<J, true, false>), kBlock, attributes)
+  CKL_SINGLE_ENTRY(linear_mfma##J##x1_deferred, LinearArgs, (linear_mfma_body<J, false, false>), kBlock, attributes) \
+  CKL_SINGLE_ENTRY(linear_mfma##J##x1_nt_deferred, LinearArgs, (linear_mfma_body<J, true, false>), kBlock, attributes)
 CKL_LINEAR_MFMA(1, )
 CKL_LINEAR_MFMA(2, )
 CKL_LINEAR_MFMA(4, CKL_TWO_WAVES)
@@ -996,6 +1001,176 @@ CKL_LINEAR_SHARED(2, 2)
 CKL_LINEAR_SHARED(2, 3)
 CKL_LINEAR_SHARED(4, 2)
 CKL_LINEAR_SHARED(4, 3)
+
+// ------------------------------------------------------------------ linear, 2 to 16 batch rows
+// The same streaming contraction over 16 batch rows with v_mfma_f32_16x16x4f32: lane (m, s) =
+// (lane & 15, lane >> 4) holds x[m][k + 4s .. k + 4s + 3] and J consecutive weight columns of the
+// rows k + 4s + i, so one wave owns a 16 x 16J tile, a wave load covers 4 weight rows and a stage
+// 16*S reduction rows. A weight feeds 16 rows instead of 32, half the MFMA time per byte. Bound by
+// the weight stream and the launch's ramp: the projections of a 4-layer decoder of 8 rows, width
+// 2048, took 753 us row-parallel and 265 us here for 806 MB of weights in 35 launches; stages of 32
+// rows (S = 2) or J = 1 were slower (283-330 and 485 us), as were more than 256 workgroups.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+template <int J, int S, int M> struct MfmaStage16 {
+  float x[S][4];
+  float w[M][S][4][J];
+};
+template <int J, int S, int M, bool Tail, bool NT>
+__device__ __forceinline__ void mfma16_load(MfmaStage16<J, S, M> &st, const float *xr, const float *const (&w)[M], long O,
+                                            int k, int k1, bool dead = false, const float *zero = nullptr) {
+#pragma unroll
+  for (int u = 0; u < S; ++u) {
+    const int kk = k + 16 * u;
+    if constexpr (!Tail) {
+      const float4 v = load4<false>(dead ? zero : xr + kk);
+      st.x[u][0] = v.x; st.x[u][1] = v.y; st.x[u][2] = v.z; st.x[u][3] = v.w;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (Tail) {
+        const bool inside = kk + i < k1;
+        const int kr = min(kk + i, k1 - 1);
+        st.x[u][i] = inside ? xr[kr] : 0.f;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          float c[J];
+          load_columns<J, NT>(c, w[m] + long(kr) * O);
+#pragma unroll
+          for (int j = 0; j < J; ++j) st.w[m][u][i][j] = inside ? c[j] : 0.f;
+        }
+      } else {
+#pragma unroll
+        for (int m = 0; m < M; ++m) load_columns<J, NT>(st.w[m][u][i], dead ? zero : w[m] + long(kk + i) * O);
+      }
+    }
+  }
+}
+// A tile has four accumulators a column, two for each of the two stage buffers, added at the end:
+// each sums a quarter of a wave's rows, so sums are as short as the row-parallel kernel's 64 rows
+// (one accumulator: error against 64 bits 1.6 times that kernel's in an MLP of 8 x 2048 x 5632).
+template <int J, int S, int M>
+__device__ __forceinline__ void mfma16_compute(const MfmaStage16<J, S, M> &st, floatx4 (&acc)[2][M][J]) {
+#pragma unroll
+  for (int u = 0; u < S; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          acc[i & 1][m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.x[u][i], st.w[m][u][i][j], acc[i & 1][m][j], 0, 0, 0);
+}
+template <int J, int S, int M, bool NT, bool Combine>
+__device__ void linear_mfma16(const LinearArgs *a, int block, float *smem) {
+  const LinearArgs &a0 = a[0];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, s = lane >> 4;
+  const int tn = block % a0.tilesN, kg = block / a0.tilesN;
+  const bool colOk = tn * 16 * J + J * m < a0.O;
+  const int n = min(tn * 16 * J + J * m, a0.O - J);   // the last lane moves back into the row, as above
+  const float *xr = a0.x + long(m < a0.B ? m : 0) * a0.I;
+  const float *w[M];
+#pragma unroll
+  for (int e = 0; e < M; ++e) w[e] = a[e].w + long(a0.layer) * a0.I * a0.O + (colOk ? n : 0);
+  const int kb0 = min(kg * a0.kChunk, a0.I), kb1 = min(kb0 + a0.kChunk, a0.I);
+  floatx4 acc[2][M][J], other[2][M][J];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int e = 0; e < M; ++e)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[h][e][j] = other[h][e][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // Stages dealt round-robin to the 4 waves and double-buffered, as in linear_mfma.
+  constexpr int R = 16 * S;
+  const int fullTotal = (kb1 - kb0) / R;
+  const int full = fullTotal > wave ? (fullTotal - wave + 3) / 4 : 0;
+  const int k = kb0 + R * wave + 4 * s;
+  const long O = a0.O;
+  MfmaStage16<J, S, M> sa, sb;
+  int t = 0;
+  if (full > 0) mfma16_load<J, S, M, false, NT>(sa, xr, w, O, k, kb1);
+  for (; t + 1 < full; t += 2) {
+    mfma16_load<J, S, M, false, NT>(sb, xr, w, O, k + 4 * R * (t + 1), kb1);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma16_compute<J, S, M>(sa, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma16_load<J, S, M, false, NT>(sa, xr, w, O, k + 4 * R * min(t + 2, full - 1), kb1, t + 2 >= full,
+                                    reinterpret_cast<const float *>(a0.workspace));
+    __builtin_amdgcn_sched_barrier(0);
+    mfma16_compute<J, S, M>(sb, other);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (t < full) mfma16_compute<J, S, M>(sa, acc);
+  const int tailBase = kb0 + R * fullTotal;
+  const int tailStages = (kb1 - tailBase + 15) / 16;
+#pragma unroll 1
+  for (int q = (wave - fullTotal % 4 + 4) % 4; q < tailStages; q += 4) {
+    MfmaStage16<J, 1, M> st;
+    mfma16_load<J, 1, M, true, NT>(st, xr, w, O, tailBase + 16 * q + 4 * s, kb1);
+    mfma16_compute<J, 1, M>(st, acc);
+  }
+
+  // The waves' accumulators meet in LDS by register; wave r adds register r of every member and
+  // column in wave order (its rows 4s + r) and stores the lane's J columns with one vector store.
+  // Planes hold the B batch rows only.
+#pragma unroll
+  for (int e = 0; e < M; ++e)
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        smem[((wave * 4 + r) * M * J + e * J + j) * 64 + lane] =
+            (acc[0][e][j][r] + acc[1][e][j][r]) + (other[0][e][j][r] + other[1][e][j][r]);
+  __syncthreads();
+  const int i = 4 * s + wave;
+#pragma unroll
+  for (int e = 0; e < M; ++e) {
+    const LinearArgs &ae = a[e];
+    float v[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      v[j] = smem[(wave * M * J + e * J + j) * 64 + lane];
+#pragma unroll
+      for (int o = 1; o < 4; ++o) v[j] += smem[((o * 4 + wave) * M * J + e * J + j) * 64 + lane];
+    }
+    const bool coherent = Combine && ae.kSplit > 1 && !ae.deferred;
+    if (colOk && i < ae.B) {
+      float *p = (ae.kSplit > 1 ? ae.partials + long(kg) * ae.B * O : ae.dst) + long(i) * O + n;
+      if (coherent) partial_store_columns<J>(p, v, (O & 1) == 0);
+      else store_columns<J>(p, v);
+    }
+    if constexpr (Combine) {
+      if (coherent && split_arrive(split_counters(ae) + tn, ae.kSplit))
+        split_finish<2>(ae, ae.partials, long(ae.B) * O, 0, 16, tn * 16 * J, 16 * J);
+    }
+  }
+}
+// ckl_linear_mfma16_<J>x1[_nt][_deferred][_shared<M>], as the 32-row entries above.
+template <int J, bool NT, bool Combine> __device__ void linear_mfma16_body(const LinearArgs &a, int block) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  linear_mfma16<J, 1, 1, NT, Combine>(&a, block, smem);
+}
+#define CKL_LINEAR_MFMA16_SHARED_ENTRY(name, J, M, NT, Combine)                                          \
+  extern "C" __global__ __launch_bounds__(kBlock) CKL_TWO_WAVES void name(const Group<LinearArgs> g) {   \
+    extern __shared__ __attribute__((aligned(16))) float smem[];                                         \
+    linear_mfma16<J, 1, M, NT, Combine>(g.m, blockIdx.x, smem);                                          \
+  }
+#define CKL_LINEAR_MFMA16_SHARED(J, M)                                                                   \
+  CKL_LINEAR_MFMA16_SHARED_ENTRY(ckl_linear_mfma16_##J##x1_shared##M, J, M, false, true)                 \
+  CKL_LINEAR_MFMA16_SHARED_ENTRY(ckl_linear_mfma16_##J##x1_nt_shared##M, J, M, true, true)               \
+  CKL_LINEAR_MFMA16_SHARED_ENTRY(ckl_linear_mfma16_##J##x1_deferred_shared##M, J, M, false, false)       \
+  CKL_LINEAR_MFMA16_SHARED_ENTRY(ckl_linear_mfma16_##J##x1_nt_deferred_shared##M, J, M, true, false)
+#define CKL_LINEAR_MFMA16(J)                                                                             \
+  CKL_ENTRY_ATTR(linear_mfma16_##J##x1, LinearArgs, (linear_mfma16_body<J, false, true>), kBlock, CKL_TWO_WAVES)      \
+  CKL_ENTRY_ATTR(linear_mfma16_##J##x1_nt, LinearArgs, (linear_mfma16_body<J, true, true>), kBlock, CKL_TWO_WAVES)    \
+  CKL_SINGLE_ENTRY(linear_mfma16_##J##x1_deferred, LinearArgs, (linear_mfma16_body<J, false, false>), kBlock, CKL_TWO_WAVES) \
+  CKL_SINGLE_ENTRY(linear_mfma16_##J##x1_nt_deferred, LinearArgs, (linear_mfma16_body<J, true, false>), kBlock, CKL_TWO_WAVES) \
+  CKL_LINEAR_MFMA16_SHARED(J, 2)                                                                         \
+  CKL_LINEAR_MFMA16_SHARED(J, 3)
+CKL_LINEAR_MFMA16(2)
+CKL_LINEAR_MFMA16(4)
 
 // ------------------------------------------------------------------ rope
 // Adjacent-pair rotation at position p (workloads.py:72-85):

@@ -1006,7 +1006,7 @@ std::map<size_t, Launch> deferCombines(const Plan &plan, const std::vector<bool>
         all = listed;
       }
     }
-    const bool vector = l.name == "ckl_linear_rowvec";
+    const bool vector = l.name == "ckl_linear_rowvec" || l.name.rfind("ckl_linear_mfma16_", 0) == 0;
     const uint64_t stride = linearPlaneRows(a.B, vector) * uint64_t(a.O);
     if (!all || stride % 4) continue;
     if (!a.partials) continue;

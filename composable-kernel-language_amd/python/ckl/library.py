@@ -123,32 +123,73 @@ LINEAR_VECTOR_WAVE_ROWS = 64  # kVectorRows: reduction rows per wave
 
 LINEAR_SHARED_J1_MEMBERS = 3   # siblings from which the MFMA path tries J = 1 first
 
+# At most 16 rows: ckl_linear_mfma16_<J> (16 rows x 16*J columns per wave) reads the weights once,
+# the row-parallel kernel once per row, but the latter does not split up to 1024 reduction rows (so
+# ordinary launches combine nothing) and fuses with the row ops around it. Measured (us a launch in a
+# graph / ordinary, rows = 8, row-parallel -> MFMA): 2048 x 2048 in a 4-layer step 753 -> 262 us a
+# step; 2048 x 1024 9.4/10.2 -> 6.2/8.9, 2048 x 512 7.2/8.3 -> 5.4/8.1, 1536 x 768 7.7/8.5 -> 5.4/8.1,
+# but 1024 x 1024 6.9/7.0 -> 5.1/8.0 and 512 x 512 5.3/6.0 -> 5.0/7.6: so more reduction rows than the
+# row-parallel kernel takes unsplit, and 2 MB of weights (4 rows of 1152 x 64, ordinary, lost 1 us).
+# Expanding projections (gate/up, heads) and q/k/v groups fill
+# the chip row by row, and lose their fusion: there the weights read again for every row must be
+# worth it (one row: 2048 x 32000 equal; 8 rows of 1024 x 8192 76 -> 56 us, of 256 x 32000 71 -> 41;
+# 8 rows of 768 x 2048 48.4 -> 48.9, 2 of 512 x 8192 39.8 -> 40.9).
+# J = 4 halves the workgroups that share a column; more than 8 splits cost more planes than they
+# give (2048 x 1024: 8 splits of J = 2 6.2 us, 16 of J = 4 6.6 us).
+LINEAR_MFMA16_MIN_CHUNK = 128
+LINEAR_MFMA16_MAX_SPLIT = 8
+LINEAR_VECTOR_UNSPLIT = LINEAR_VECTOR_WAVES * LINEAR_VECTOR_WAVE_ROWS
+
+
+def _mfma_tiling(b: int, i: int, o: int, order, tile_rows: int, min_chunk: int, max_split: int):
+    """(J, column tiles, K splits, slice rows) of an MFMA linear: the first J of `order` whose grid
+    fills at least LINEAR_MIN_FILL of LINEAR_TARGET_GROUPS without exceeding it, else the fullest."""
+    row_tiles = _cdiv(b, tile_rows)
+    best = None
+    for j in order:
+        if j > o:                                  # a lane's j columns are columns of one row
+            continue
+        tiles = _cdiv(o, tile_rows * j)            # as many lanes hold columns as rows
+        split = max(1, min(LINEAR_TARGET_GROUPS // (row_tiles * tiles), i // min_chunk, max_split))
+        chunk = _cdiv(_cdiv(i, split), 16) * 16
+        split = _cdiv(i, chunk)
+        grid = row_tiles * tiles * split
+        fill = grid / LINEAR_TARGET_GROUPS if grid <= LINEAR_TARGET_GROUPS else 0.5
+        if best is None or fill > best[0]:
+            best = (fill, j, tiles, split, chunk)
+        if fill >= LINEAR_MIN_FILL:
+            return best[1:]
+    return best[1:]
+
+
+def _takes_mfma16(b: int, i: int, o: int, members: int) -> bool:
+    """Whether a linear of at most LINEAR_VECTOR_ROWS rows takes the 16-row MFMA kernel (the figures
+    are above)."""
+    weights = 4 * i * o
+    if members >= LINEAR_SHARED_J1_MEMBERS:
+        return b * weights >= 32 << 20
+    if o > i:
+        return b * weights >= 48 << 20 or (weights >= 8 << 20 and i >= LINEAR_VECTOR_UNSPLIT)
+    return i > LINEAR_VECTOR_UNSPLIT and o >= 16 and weights >= 2 << 20
+
 
 def linear_tiling(b: int, i: int, o: int, members: int = 1) -> dict:
     """Tiling of one linear (`members` = how many sibling linears of this shape multiply the same
     x and run as one shared-operand launch)."""
+    block = BLOCK
     if b > LINEAR_VECTOR_ROWS:
+        order = (1, 2, 4) if members >= LINEAR_SHARED_J1_MEMBERS else (2, 4, 1)
+        j, tiles, split, chunk = _mfma_tiling(b, i, o, order, 32, LINEAR_MIN_CHUNK, LINEAR_TARGET_GROUPS)
         row_tiles = _cdiv(b, 32)
-        best = None
-        for j in ((1, 2, 4) if members >= LINEAR_SHARED_J1_MEMBERS else (2, 4, 1)):
-            if j > o:                                  # a lane's j columns are columns of one row
-                continue
-            tiles = _cdiv(o, 32 * j)
-            split = max(1, min(LINEAR_TARGET_GROUPS // (row_tiles * tiles), i // LINEAR_MIN_CHUNK))
-            chunk = _cdiv(_cdiv(i, split), 16) * 16
-            split = _cdiv(i, chunk)
-            grid = row_tiles * tiles * split
-            fill = grid / LINEAR_TARGET_GROUPS if grid <= LINEAR_TARGET_GROUPS else 0.5
-            if best is None or fill > best[0]:
-                best = (fill, j, tiles, split, chunk)
-            if fill >= LINEAR_MIN_FILL:
-                best = (fill, j, tiles, split, chunk)
-                break
-        _, j, tiles, split, chunk = best
         rows = row_tiles * 32
         shared = j * LINEAR_EPILOGUE_COLUMN_BYTES      # the 4 waves' accumulator tiles, one pass
         entry = f"ckl_linear_mfma{j}x1"
-        block = BLOCK
+    elif _takes_mfma16(b, i, o, members):
+        order = (2, 4) if members >= LINEAR_SHARED_J1_MEMBERS else (4, 2)
+        j, tiles, split, chunk = _mfma_tiling(b, i, o, order, 16, LINEAR_MFMA16_MIN_CHUNK, LINEAR_MFMA16_MAX_SPLIT)
+        row_tiles, rows = 1, b                            # planes hold the batch rows only
+        shared = j * LINEAR_EPILOGUE_COLUMN_BYTES // 4    # 4 accumulator registers a column
+        entry = f"ckl_linear_mfma16_{j}x1"
     else:
         tiles = _cdiv(o, 64)
         waves = min(LINEAR_VECTOR_WAVES, _cdiv(i, LINEAR_VECTOR_WAVE_ROWS))
@@ -160,8 +201,7 @@ def linear_tiling(b: int, i: int, o: int, members: int = 1) -> dict:
         block = 64 * waves
     workspace, partials = LINEAR_ZERO_PAGE, 0
     if split > 1:
-        counters = row_tiles * tiles if entry != "ckl_linear_rowvec" else b * tiles
-        workspace += _cdiv(4 * counters, 256) * 256
+        workspace += _cdiv(4 * row_tiles * tiles, 256) * 256
         partials = 4 * split * rows * o
     return dict(grid=row_tiles * split * tiles, tiles=tiles, split=split, chunk=chunk, shared=shared, entry=entry,
                 workspace=workspace, partials=partials, block=block)
