@@ -123,6 +123,14 @@ struct CKL_ALIGN RopeAttentionChainArgs {
   PartialSource qsrc, ksrc, v;
 };
 
+// Whether attention rows of D floats take the scores' padded vector layout (library.hip,
+// attention_scores): a multiple of 4 up to 256 that no exact layout covers.
+constexpr bool scoresPadded(int D) {
+  if (D <= 0 || (D & 3) || D > 256) return false;
+  const int P = D <= 32 ? 1 : D <= 64 ? 2 : 4, G = D / (4 * P);
+  return G * 4 * P != D || (G & (G - 1)) != 0;
+}
+
 // Entry points named <entry>_nt read their streamed operand (weights, the cache) with
 // nontemporal loads; the executor selects them when that operand is at least this large.
 constexpr int64_t kStreamBytes = int64_t(8) << 20;

@@ -1299,19 +1299,22 @@ __device__ __forceinline__ float score_scalar(const float *q, const float *key, 
 }
 // Vector layout of the scores: groups of G lanes hold one cache row, each lane P float4 pieces of
 // it (pieces part + G*j, j < P): P = 1 and G = D/4 for D <= 32, P = 2 for D <= 64, else P = 4,
-// with G = D/(4P) a power of two (8 lanes for D = 64 and 128, 16 for D = 256); other D (D = 96:
-// G = 6) take the sequential dot product. A P = 3 instantiation for D = 96 would give it 8-lane
-// groups, but it doubled the VGPRs of the rope/attention chain kernel for every D (69 -> 148,
-// with scratch), so the chain ran 40% slower at D = 128; it is not instantiated. Each lane adds its 4P products with explicit FMAs in piece order, then
-// the row is summed over its G lanes (group_sum), so with 8-lane groups a row costs three DPP
-// steps instead of a 32-lane butterfly. A wave load covers 64/G rows; a lane keeps kScoreBatch
-// pieces in flight (kScoreBatch/P rows).
+// with G = D/(4P) a power of two (8 lanes for D = 64 and 128, 16 for D = 256). Any other D that is
+// a multiple of 4 up to 256 takes P = 4 with the next power of two lanes (D = 80, 96: G = 8; D = 48:
+// G = 4): the pieces past the row re-read one of the lane's own and are replaced by zero, in an
+// instantiation of their own (Pad), so that the exact sizes spend no selects. (P = 3 for D = 96
+// would waste no piece, but doubled the VGPRs of the rope/attention chain for every D.) One thread a
+// row with a sequential dot product, which these took before, and one thread an element of the
+// values, serial over the rows: 3 requests of 7 heads of 80 at 701 rows, ordinary, scores 12.2 ->
+// 4.7 us, values 69.8 -> 5.7 us; the chain of 4 x 8 heads of 96 at 901 rows 109 -> 23.5 us. Each lane
+// adds its 4P products with explicit FMAs in piece order, then the row is summed over its G lanes
+// (group_sum), so with 8-lane groups a row costs three DPP steps instead of a 32-lane butterfly. A
+// wave load covers 64/G rows; a lane keeps kScoreBatch pieces in flight (kScoreBatch/P rows).
 __device__ __forceinline__ int score_pieces(int D) { return D <= 32 ? 1 : D <= 64 ? 2 : 4; }
-__device__ __forceinline__ bool scores_vector_layout(int D) {
-  if ((D & 3) || D > 256) return false;
-  const int P = score_pieces(D), G = D / (4 * P);
-  return G * 4 * P == D && (G & (G - 1)) == 0;        // G lanes a row: a power of two
-}
+__device__ __forceinline__ bool scores_vector_layout(int D) { return (D & 3) == 0 && D <= 256; }
+// Instantiation of the vector layout a row of D takes: its P, or 0 for the padded one (the executor
+// picks the rope chain's by scoresPadded, csrc/runtime/chains.cpp).
+__device__ __forceinline__ int score_layout(int D) { return scoresPadded(D) ? 0 : score_pieces(D); }
 // Partial dot product of a lane's P pieces of q and of one key row.
 template <int P> __device__ __forceinline__ float dot_pieces(const float4 (&q)[P], const float4 *k) {
   float v = q[0].x * k[0].x;
@@ -1327,23 +1330,60 @@ template <int P> __device__ __forceinline__ float dot_pieces(const float4 (&q)[P
   }
   return v;
 }
-template <int P> struct KeyLayout {
+// K is the layout's instantiation: P pieces a lane (1, 2, 4), or 0 for the padded one.
+template <int K> struct KeyLayout {
+  static constexpr bool Pad = K == 0;
+  static constexpr int P = Pad ? 4 : K;
   static constexpr int U = kScoreBatch / P;        // rows per lane per batch
-  int G, rowsPerLoad, sub, part;
-  __device__ explicit KeyLayout(int D) : G(D / (4 * P)), rowsPerLoad(64 / (D / (4 * P))) {
+  int G, rowsPerLoad, sub, part, pieces;
+  __device__ explicit KeyLayout(int D) {
+    pieces = D / 4;
+    if constexpr (Pad) {
+      G = 1;
+      while (G * P < pieces) G *= 2;
+    } else {
+      G = D / (4 * P);
+    }
+    rowsPerLoad = 64 / G;
     const int lane = threadIdx.x & 63;
     sub = lane / G;
     part = lane % G;
   }
   __device__ int rowsPerBatch() const { return U * rowsPerLoad; }
+  // Float offset of the lane's piece j in a row; the padded layout's lanes without a piece j read
+  // piece `part` (their own when there is one, else one that exists).
+  __device__ int offset(int j) const {
+    const int at = part + G * j;
+    if constexpr (Pad) return 4 * (at < pieces ? at : min(part, pieces - 1));
+    return 4 * at;
+  }
+  __device__ float4 keep(float4 v, int j) const {
+    if constexpr (Pad) {
+      const bool in = part + G * j < pieces;
+      return make_float4(in ? v.x : 0.f, in ? v.y : 0.f, in ? v.z : 0.f, in ? v.w : 0.f);
+    }
+    return v;
+  }
   template <typename T> __device__ void loadQuery(float4 (&qv)[P], const T *q) const {
 #pragma unroll
-    for (int j = 0; j < P; ++j) qv[j] = reinterpret_cast<const float4 *>(q)[part + G * j];
+    for (int j = 0; j < P; ++j) qv[j] = keep(*reinterpret_cast<const float4 *>(q + offset(j)), j);
+  }
+  // Partial dot product of the lane's pieces of the query and of one loaded key row.
+  __device__ float dot(const float4 (&qv)[P], const float4 *kv) const {
+    if constexpr (Pad) {
+      float4 k[P];
+#pragma unroll
+      for (int j = 0; j < P; ++j) k[j] = keep(kv[j], j);
+      return dot_pieces<P>(qv, k);
+    } else {
+      return dot_pieces<P>(qv, kv);
+    }
   }
 };
-template <bool NT, int P> __device__ void attention_scores_rows(const ScoresArgs &a, const float *q, const float *keys,
+template <bool NT, int K> __device__ void attention_scores_rows(const ScoresArgs &a, const float *q, const float *keys,
                                                           float *scores, int w0, int w1) {
-  const KeyLayout<P> k(a.D);
+  constexpr int P = KeyLayout<K>::P;
+  const KeyLayout<K> k(a.D);
   float4 qv[P];
   k.loadQuery(qv, q);
   for (int base = w0; base < w1; base += k.rowsPerBatch()) {
@@ -1353,11 +1393,11 @@ template <bool NT, int P> __device__ void attention_scores_rows(const ScoresArgs
       int t = base + u * k.rowsPerLoad + k.sub;
       t = t < w1 ? t : min(w0 + k.sub, w1 - 1);    // past the end: re-read an early row, dropped
 #pragma unroll
-      for (int j = 0; j < P; ++j) kv[u * P + j] = load4<NT>(keys + long(t) * a.D + 4 * (k.part + k.G * j));
+      for (int j = 0; j < P; ++j) kv[u * P + j] = load4<NT>(keys + long(t) * a.D + k.offset(j));
     }
 #pragma unroll
     for (int u = 0; u < k.U; ++u) {
-      float v = group_sum(dot_pieces<P>(qv, kv + u * P), k.G);
+      float v = group_sum(k.dot(qv, kv + u * P), k.G);
       int t = base + u * k.rowsPerLoad + k.sub;
       if (k.part == 0 && t < w1) scores[t] = v * a.scale;
     }
@@ -1379,7 +1419,8 @@ template <bool NT> __device__ void attention_scores_body(const ScoresArgs &a, in
   if (scores_vector_layout(a.D)) {
     const int wave = threadIdx.x >> 6;
     const int w0 = t0 + wave * 64, w1 = min(w0 + 64, tEnd);
-    switch (score_pieces(a.D)) {
+    switch (score_layout(a.D)) {
+      case 0: attention_scores_rows<NT, 0>(a, q, keys, scores, w0, w1); break;
       case 1: attention_scores_rows<NT, 1>(a, q, keys, scores, w0, w1); break;
       case 2: attention_scores_rows<NT, 2>(a, q, keys, scores, w0, w1); break;
       default: attention_scores_rows<NT, 4>(a, q, keys, scores, w0, w1); break;
@@ -1483,7 +1524,9 @@ CKL_ENTRY(softmax, SoftmaxArgs, softmax_body)
 // sums are combined by a fixed-order tree in LDS. `probs` is the (b, h) row of probabilities
 // (global memory, or LDS in the softmax chain).
 constexpr int kValuesBatch = 8;
-__device__ __forceinline__ bool values_vector_layout(int D) { return (D & 3) == 0 && D <= 4 * 64 && (64 % (D / 4)) == 0; }
+// Groups of D/4 lanes own one row's float4s; blockDim / (D/4) groups fit the workgroup, the threads
+// past the last group (D/4 not a divisor of the workgroup, D = 48, 80, 96) only synchronize.
+__device__ __forceinline__ bool values_vector_layout(int D) { return (D & 3) == 0 && D <= 4 * 64; }
 // A thread's kValuesBatch cache-row loads of the values' vector layout, rows base + u*groups + g
 // (rows past `end` re-read an early row; end > 0).
 struct ValueBatch { float4 v[kValuesBatch]; };
@@ -1501,54 +1544,66 @@ __device__ __forceinline__ void load_value_batch(ValueBatch &vb, const float *va
 __device__ __forceinline__ const float *values_slab(const ValuesArgs &a, long bh) {
   return a.vc + (long(a.layer) * a.B * a.A + bh) * long(a.T) * a.D;
 }
+// Sum over rows [t0, end) of probs[t] * values[t, :] in the vector layout; the threads of group 0
+// (threadIdx.x < D/4) return their float4 of it. `haveFirst`: `first` holds this thread's first
+// batch (t0 = 0, end > 0). The groups' sums are added by a fixed-order tree in LDS.
+template <bool NT>
+__device__ __forceinline__ float4 values_reduce(const float *values, int D, const float *probs, int t0, int end,
+                                                const ValueBatch &first, bool haveFirst) {
+  __shared__ float4 partial[kValuesBlock];
+  const int width = D / 4, groups = int(blockDim.x) / width;
+  const int g = threadIdx.x / width;
+  const int step = kValuesBatch * groups;
+  const int stop = g < groups ? end : 0;             // threads past the last group add nothing
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto consume = [&](const ValueBatch &vb, int base) {
+#pragma unroll
+    for (int u = 0; u < kValuesBatch; ++u) {
+      int t = base + u * groups + g;
+      int tc = t < end ? t : min(g, end - 1);
+      float pr = t < stop ? probs[tc] : 0.f;
+      acc.x = __builtin_fmaf(pr, vb.v[u].x, acc.x);
+      acc.y = __builtin_fmaf(pr, vb.v[u].y, acc.y);
+      acc.z = __builtin_fmaf(pr, vb.v[u].z, acc.z);
+      acc.w = __builtin_fmaf(pr, vb.v[u].w, acc.w);
+    }
+  };
+  int base = t0;
+  if (haveFirst) {
+    consume(first, 0);
+    base = step;
+  }
+  for (; base < end; base += step) {
+    ValueBatch vb;
+    load_value_batch<NT>(vb, values, D, base, end);
+    consume(vb, base);
+  }
+  partial[threadIdx.x] = acc;
+  __syncthreads();
+  int stride = 1;
+  while (2 * stride < groups) stride *= 2;           // half the groups, rounded up to a power of two
+  for (; stride > 0 && groups > 1; stride /= 2) {
+    if (g < stride && g + stride < groups) {
+      float4 o = partial[threadIdx.x + stride * width];
+      float4 s = partial[threadIdx.x];
+      partial[threadIdx.x] = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
+    }
+    __syncthreads();
+  }
+  return partial[threadIdx.x % width];
+}
 // `haveFirst`: `first` holds this thread's first batch (vector layout, end > 0). `p` is the
 // position (a.position[0]), loaded by the caller.
 template <bool NT>
 __device__ __forceinline__ void attention_values_row(const ValuesArgs &a, long bh, const float *probs,
                                                      const ValueBatch &first, bool haveFirst, int p) {
-  __shared__ float4 partial[kValuesBlock];
   int end = min(p + 1, a.T);
   if (p < 0) end = 0;
   const float *values = values_slab(a, bh);
   float *dst = a.dst + bh * a.D;
   if (values_vector_layout(a.D)) {
-    const int width = a.D / 4, groups = int(blockDim.x) / width;
-    const int g = threadIdx.x / width, part = threadIdx.x % width;
-    const int step = kValuesBatch * groups;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto consume = [&](const ValueBatch &vb, int base) {
-#pragma unroll
-      for (int u = 0; u < kValuesBatch; ++u) {
-        int t = base + u * groups + g;
-        int tc = t < end ? t : min(g, end - 1);
-        float pr = t < end ? probs[tc] : 0.f;
-        acc.x = __builtin_fmaf(pr, vb.v[u].x, acc.x);
-        acc.y = __builtin_fmaf(pr, vb.v[u].y, acc.y);
-        acc.z = __builtin_fmaf(pr, vb.v[u].z, acc.z);
-        acc.w = __builtin_fmaf(pr, vb.v[u].w, acc.w);
-      }
-    };
-    int base = 0;
-    if (haveFirst) {
-      consume(first, 0);
-      base = step;
-    }
-    for (; base < end; base += step) {
-      ValueBatch vb;
-      load_value_batch<NT>(vb, values, a.D, base, end);
-      consume(vb, base);
-    }
-    partial[threadIdx.x] = acc;
-    __syncthreads();
-    for (int stride = groups / 2; stride > 0; stride /= 2) {
-      if (g < stride) {
-        float4 o = partial[threadIdx.x + stride * width];
-        float4 s = partial[threadIdx.x];
-        partial[threadIdx.x] = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
-      }
-      __syncthreads();
-    }
-    if (g == 0) reinterpret_cast<float4 *>(dst)[part] = partial[part];
+    const float4 sum = values_reduce<NT>(values, a.D, probs, 0, end, first, haveFirst);
+    if (int(threadIdx.x) < a.D / 4) reinterpret_cast<float4 *>(dst)[threadIdx.x] = sum;
   } else {
     for (int d = threadIdx.x; d < a.D; d += blockDim.x) {
       float acc = 0.f;
@@ -1597,23 +1652,25 @@ CKL_ENTRY_ATTR(softmax__attention_values_nt, SoftmaxValuesChainArgs, softmax__at
 // A wave's batch of cache-row loads in the scores' vector layout (KeyLayout<P>): rows
 // base + u*rowsPerLoad + sub for u < U, P pieces each; rows past `end` re-read an early row.
 struct KeyBatch { float4 kv[kScoreBatch]; };
-template <bool NT, int P>
-__device__ __forceinline__ void load_key_batch(KeyBatch &kb, const float *keys, int D, const KeyLayout<P> &k, int base,
+template <bool NT, int K>
+__device__ __forceinline__ void load_key_batch(KeyBatch &kb, const float *keys, int D, const KeyLayout<K> &k, int base,
                                                int end) {
+  constexpr int P = KeyLayout<K>::P;
 #pragma unroll
   for (int u = 0; u < k.U; ++u) {
     int t = base + u * k.rowsPerLoad + k.sub;
     t = t < end ? t : min(k.sub, end - 1);        // past the end: re-read an early row, dropped
 #pragma unroll
-    for (int j = 0; j < P; ++j) kb.kv[u * P + j] = load4<NT>(keys + long(t) * D + 4 * (k.part + k.G * j));
+    for (int j = 0; j < P; ++j) kb.kv[u * P + j] = load4<NT>(keys + long(t) * D + k.offset(j));
   }
 }
-template <int P>
-__device__ __forceinline__ void score_key_batch(const KeyBatch &kb, const float4 (&qv)[P], const KeyLayout<P> &k, int base,
-                                                int end, float scale, float *rowScores, float *scores) {
+template <int K>
+__device__ __forceinline__ void score_key_batch(const KeyBatch &kb, const float4 (&qv)[KeyLayout<K>::P], const KeyLayout<K> &k,
+                                                int base, int end, float scale, float *rowScores, float *scores) {
+  constexpr int P = KeyLayout<K>::P;
 #pragma unroll
   for (int u = 0; u < k.U; ++u) {
-    float v = group_sum(dot_pieces<P>(qv, kb.kv + u * P), k.G) * scale;
+    float v = group_sum(k.dot(qv, kb.kv + u * P), k.G) * scale;
     int t = base + u * k.rowsPerLoad + k.sub;
     if (k.part == 0 && t < end) {
       rowScores[t] = v;
@@ -1629,7 +1686,7 @@ __device__ __forceinline__ void score_key_batch(const KeyBatch &kb, const float4
 // `appended` (the rope chain, position in range), the key row at the position is read from LDS
 // instead of the cache and `storesPending` waves wait for their cache-row stores before the
 // barrier that precedes the values. The first batch of value rows is loaded before the softmax.
-template <bool NT, int P>
+template <bool NT, int K>
 __device__ __forceinline__ void attention_chain_row(const ScoresArgs &sc, const SoftmaxArgs &softmax,
                                                     const ValuesArgs &values, long bh, const float *q, int p,
                                                     float *rowScores, const KeyBatch &first, bool haveFirst,
@@ -1640,7 +1697,8 @@ __device__ __forceinline__ void attention_chain_row(const ScoresArgs &sc, const 
   float *scores = sc.scores ? sc.scores + bh * sc.T : nullptr;
   const bool vector = scores_vector_layout(sc.D);
   if (vector) {
-    const KeyLayout<P> k(sc.D);
+    constexpr int P = KeyLayout<K>::P;
+    const KeyLayout<K> k(sc.D);
     const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     float4 qv[P];
     k.loadQuery(qv, q);
@@ -1648,19 +1706,19 @@ __device__ __forceinline__ void attention_chain_row(const ScoresArgs &sc, const 
     const int endG = appended ? end - 1 : end;       // the appended row comes from LDS
     int base = wave * k.rowsPerBatch();
     if (haveFirst) {
-      score_key_batch(first, qv, k, base, endG, sc.scale, rowScores, scores);
+      score_key_batch<K>(first, qv, k, base, endG, sc.scale, rowScores, scores);
       base += step;
     }
     for (; base < endG; base += step) {
       KeyBatch kb;
-      load_key_batch<NT, P>(kb, keys, sc.D, k, base, endG);
-      score_key_batch(kb, qv, k, base, endG, sc.scale, rowScores, scores);
+      load_key_batch<NT, K>(kb, keys, sc.D, k, base, endG);
+      score_key_batch<K>(kb, qv, k, base, endG, sc.scale, rowScores, scores);
     }
     if (appended && wave == 0) {
       // The row's score with the arithmetic of the cache path (any lane group reduces alike).
       float4 kv[P];
       k.loadQuery(kv, appended);
-      float v = group_sum(dot_pieces<P>(qv, kv), k.G) * sc.scale;
+      float v = group_sum(k.dot(qv, kv), k.G) * sc.scale;
       if ((threadIdx.x & 63) == 0) {
         rowScores[p] = v;
         if (scores) scores[p] = v;
@@ -1692,7 +1750,8 @@ __device__ void attention_scores__softmax__attention_values_body(const Attention
   KeyBatch none;
   const float *q = a.scores.q + bh * a.scores.D;
   const int p = load_position(a.scores.position);
-  switch (score_pieces(a.scores.D)) {
+  switch (score_layout(a.scores.D)) {
+    case 0: attention_chain_row<NT, 0>(a.scores, a.softmax, a.values, bh, q, p, rowScores, none, false); break;
     case 1: attention_chain_row<NT, 1>(a.scores, a.softmax, a.values, bh, q, p, rowScores, none, false); break;
     case 2: attention_chain_row<NT, 2>(a.scores, a.softmax, a.values, bh, q, p, rowScores, none, false); break;
     default: attention_chain_row<NT, 4>(a.scores, a.softmax, a.values, bh, q, p, rowScores, none, false); break;
@@ -1737,7 +1796,7 @@ __device__ __forceinline__ float2 sum_pair(const PartialSource &src, const float
   }
   return t;
 }
-template <bool NT, int P>
+template <bool NT, int K>
 __device__ void rope_attention_rows(const RopeAttentionChainArgs &a, int block) {
   extern __shared__ float rowScores[];
   const RopeArgs &q = a.q, &k = a.k;
@@ -1754,7 +1813,7 @@ __device__ void rope_attention_rows(const RopeAttentionChainArgs &a, int block) 
   // launch writes only row p of the cache.
   const int wave = threadIdx.x >> 6;
   const bool vector = scores_vector_layout(sc.D);
-  const KeyLayout<P> layout(vector ? sc.D : 4 * P);
+  const KeyLayout<K> layout(vector ? sc.D : 4 * KeyLayout<K>::P);
   const int firstBase = wave * layout.rowsPerBatch();
   const bool early = vector && inRange && p >= 1;
   // With one pair a thread and at most kRopeRequest planes a source, a thread's rotation operands
@@ -1774,7 +1833,7 @@ __device__ void rope_attention_rows(const RopeAttentionChainArgs &a, int block) 
   }
   KeyBatch first;
   if (early)
-    load_key_batch<NT, P>(first, sc.kc + (long(sc.layer) * sc.B * sc.A + bh) * long(sc.T) * sc.D, sc.D, layout,
+    load_key_batch<NT, K>(first, sc.kc + (long(sc.layer) * sc.B * sc.A + bh) * long(sc.T) * sc.D, sc.D, layout,
                           firstBase, p);
   if (requestFirst) {
     if (pair < q.R) {
@@ -1815,7 +1874,7 @@ __device__ void rope_attention_rows(const RopeAttentionChainArgs &a, int block) 
   __syncthreads();
   // The barrier alone does not wait for vector stores: the waves that appended cache rows wait for
   // them before the barrier that precedes the values (the scores take the key row from LDS).
-  attention_chain_row<NT, P>(a.scores, a.softmax, a.values, bh, inRange ? qrow : sc.q + bh * sc.D, p, rowScores,
+  attention_chain_row<NT, K>(a.scores, a.softmax, a.values, bh, inRange ? qrow : sc.q + bh * sc.D, p, rowScores,
                              first, early, inRange ? krow : nullptr, inRange && int(threadIdx.x & ~63) < q.R);
 }
 template <bool NT> __device__ void rope_attention_stream(const RopeAttentionChainArgs &a, int block) {
@@ -1829,6 +1888,13 @@ CKL_ENTRY_ATTR(rope__rope__append_kv__attention_scores__softmax__attention_value
                rope_attention_stream<false>, kValuesBlock, )
 CKL_ENTRY_ATTR(rope__rope__append_kv__attention_scores__softmax__attention_values_nt, RopeAttentionChainArgs,
                rope_attention_stream<true>, kValuesBlock, )
+// Head sizes of the scores' padded layout have entries of their own: a fourth instantiation in the
+// kernel above took it from 93 to 148-162 VGPRs with scratch. Its scalar path (D % 4 != 0 or
+// D > 256) stays above.
+CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores__softmax__attention_values_padded, RopeAttentionChainArgs,
+                 (rope_attention_rows<false, 0>), kValuesBlock, )
+CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores__softmax__attention_values_padded_nt, RopeAttentionChainArgs,
+                 (rope_attention_rows<true, 0>), kValuesBlock, )
 
 // ------------------------------------------------------------------ pointwise
 // add: dst = x + y; multiply: dst = x * y; silu: dst = v / (1 + exp(-v)) (workloads.py:145-167).

@@ -849,8 +849,17 @@ std::vector<Chain> findChains(const Plan &plan, const std::vector<bool> &tempora
         trace(head, rule, "the code object has no such entry point");
         continue;
       }
-      // A chain with a streaming member runs its nontemporal-load variant when there is one.
       std::string entry = rule.entry;
+      // The rope/attention chain has an entry of its own for head sizes of the scores' padded layout.
+      if (rule.build == ropeAttentionChain && scoresPadded(block<ScoresArgs>(plan.nodes[roles[3]].launch).D)) {
+        entry += "_padded";
+        if (hipModuleGetFunction(&function, first.module, entry.c_str()) != hipSuccess) {
+          (void)hipGetLastError();
+          trace(head, rule, "the code object has no entry point for this head size");
+          continue;
+        }
+      }
+      // A chain with a streaming member runs its nontemporal-load variant when there is one.
       bool streaming = false;
       for (size_t m : roles) streaming |= streams(plan.nodes[m].launch);
       if (streaming) {

@@ -264,8 +264,8 @@ def _values(shapes, consts, ext):
     if a * d != c or not (0 <= layer < l) or not (ext[0] >= d and ext[1:] == (a, b)):
         return None
     # Enough row groups to keep ~8 rows in flight per lane over the whole capacity, at least one
-    # wave, at most VALUES_BLOCK threads; the D/4 lanes of a row must divide a wave.
-    width = d // 4 if d % 4 == 0 and d <= 256 and 64 % (d // 4) == 0 else 64
+    # wave, at most VALUES_BLOCK threads; D/4 lanes own a row.
+    width = d // 4 if d % 4 == 0 and d <= 256 else 64
     block = 64
     while block < VALUES_BLOCK and (block // width) * 8 < t:
         block *= 2
