@@ -130,10 +130,11 @@ LINEAR_SHARED_J1_MEMBERS = 3   # siblings from which the MFMA path tries J = 1 f
 # step; 2048 x 1024 9.4/10.2 -> 6.2/8.9, 2048 x 512 7.2/8.3 -> 5.4/8.1, 1536 x 768 7.7/8.5 -> 5.4/8.1,
 # but 1024 x 1024 6.9/7.0 -> 5.1/8.0 and 512 x 512 5.3/6.0 -> 5.0/7.6: so more reduction rows than the
 # row-parallel kernel takes unsplit, and 2 MB of weights (4 rows of 1152 x 64, ordinary, lost 1 us).
-# Expanding projections (gate/up, heads) and q/k/v groups fill
-# the chip row by row, and lose their fusion: there the weights read again for every row must be
-# worth it (one row: 2048 x 32000 equal; 8 rows of 1024 x 8192 76 -> 56 us, of 256 x 32000 71 -> 41;
-# 8 rows of 768 x 2048 48.4 -> 48.9, 2 of 512 x 8192 39.8 -> 40.9).
+# q/k/v groups need both that and 32 MB read for all rows (8 rows of 1024 x 1024, ordinary: a layer
+# 46.1 -> 50.6 us). Expanding projections (gate/up, heads) fill the chip row by row and lose their
+# fusion: there the weights read again for every row must be worth it (one row: 2048 x 32000 equal;
+# 8 rows of 1024 x 8192 76 -> 56 us, of 256 x 32000 71 -> 41; 8 rows of 768 x 2048 48.4 -> 48.9, 2 of
+# 512 x 8192 39.8 -> 40.9).
 # J = 4 halves the workgroups that share a column; more than 8 splits cost more planes than they
 # give (2048 x 1024: 8 splits of J = 2 6.2 us, 16 of J = 4 6.6 us).
 LINEAR_MFMA16_MIN_CHUNK = 128
@@ -167,7 +168,7 @@ def _takes_mfma16(b: int, i: int, o: int, members: int) -> bool:
     are above)."""
     weights = 4 * i * o
     if members >= LINEAR_SHARED_J1_MEMBERS:
-        return b * weights >= 32 << 20
+        return i > LINEAR_VECTOR_UNSPLIT and b * weights >= 32 << 20
     if o > i:
         return b * weights >= 48 << 20 or (weights >= 8 << 20 and i >= LINEAR_VECTOR_UNSPLIT)
     return i > LINEAR_VECTOR_UNSPLIT and o >= 16 and weights >= 2 << 20
