@@ -78,6 +78,14 @@ struct CKL_ALIGN ScoresArgs { const float *q; const float *kc; const int *positi
 struct CKL_ALIGN SoftmaxArgs { const float *scores; const int *position; float *probs; int B, A, T, rowThreads; };
 // dst[b, h*D+d] = sum_t probs[b, h, t] * vc[layer, b, h, t, d]   (workloads.py:131-142)
 struct CKL_ALIGN ValuesArgs { const float *probs; const float *vc; const int *position; float *dst; int L, B, A, T, D, layer; };
+// attention_values with the cache rows of a (b, h) cut into `slices` runs of workgroups
+// (ckl_attention_values_split). `workspace`: a completion counter per (b, h), reset by the last
+// slice; `partials`: float[B * A][slices][D].
+struct CKL_ALIGN ValuesSplitArgs {
+  const float *probs; const float *vc; const int *position; float *dst; int L, B, A, T, D, layer, slices;
+  unsigned char *workspace;
+  float *partials;
+};
 // add / multiply / silu over n elements   (workloads.py:145-167)
 struct CKL_ALIGN BinaryArgs { const float *x; const float *y; float *dst; int n; };
 struct CKL_ALIGN UnaryArgs { const float *src; float *dst; int n; };

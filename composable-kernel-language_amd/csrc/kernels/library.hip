@@ -1434,15 +1434,15 @@ CKL_ENTRY(attention_scores_nt, ScoresArgs, attention_scores_body<true>)
 
 // ------------------------------------------------------------------ softmax
 // probs[b,h,t] = exp(s[t] - max) / sum_t' exp(s[t'] - max) over t <= p (workloads.py:114-128).
-// `rowThreads` (64 or 256) lanes per (b, h) row; each lane keeps up to kSoftmaxPerLane scores in
+// `rowThreads` (64, 256 or 1024) lanes per (b, h) row; each lane keeps up to kSoftmaxPerLane scores in
 // registers (one read of the row, one write), longer rows stream three passes.
 constexpr int kSoftmaxPerLane = 8;
 constexpr int kValuesBlock = 512;
 
-// Reduction over the `rowThreads` lanes of one row (a wave, or waves 0-3 of the workgroup). With
+// Reduction over the `rowThreads` lanes of one row (a wave, or the first waves of the workgroup). With
 // rowThreads > 64 every thread of the workgroup must call it (it synchronizes the workgroup).
 template <bool IsMax> __device__ __forceinline__ float row_reduce(float v, int rowThreads) {
-  __shared__ float across[kValuesBlock / 64];
+  __shared__ float across[16];
   v = IsMax ? wave_max(v) : wave_sum(v);
   if (rowThreads <= 64) return v;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1450,7 +1450,7 @@ template <bool IsMax> __device__ __forceinline__ float row_reduce(float v, int r
   if (lane == 0) across[wave] = v;
   __syncthreads();
   float r = across[0];
-  for (int w = 1; w < kBlock / 64; ++w) r = IsMax ? fmaxf(r, across[w]) : r + across[w];
+  for (int w = 1; w < rowThreads / 64; ++w) r = IsMax ? fmaxf(r, across[w]) : r + across[w];
   return r;
 }
 
@@ -1508,13 +1508,13 @@ __device__ __forceinline__ void softmax_row(const SoftmaxArgs &a, const float *s
 }
 
 __device__ void softmax_body(const SoftmaxArgs &a, int block) {
-  const int rowsPerBlock = kBlock / a.rowThreads;
+  const int rowsPerBlock = int(blockDim.x) / a.rowThreads;
   const int local = threadIdx.x % a.rowThreads;
   long row = long(block) * rowsPerBlock + threadIdx.x / a.rowThreads;
   const bool active = row < long(a.B) * a.A;       // uniform per row group (rowThreads divides kBlock)
   softmax_row(a, a.scores + (active ? row : 0) * a.T, row, local, active, nullptr, load_position(a.position));
 }
-CKL_ENTRY(softmax, SoftmaxArgs, softmax_body)
+CKL_ENTRY_ATTR(softmax, SoftmaxArgs, softmax_body, 1024, )
 
 // ------------------------------------------------------------------ attention_values
 // dst[b, h*D+d] = sum_{t<=p} probs[b,h,t] * vc[layer,b,h,t,d]   (workloads.py:131-142).
@@ -1543,6 +1543,24 @@ __device__ __forceinline__ void load_value_batch(ValueBatch &vb, const float *va
 }
 __device__ __forceinline__ const float *values_slab(const ValuesArgs &a, long bh) {
   return a.vc + (long(a.layer) * a.B * a.A + bh) * long(a.T) * a.D;
+}
+// The row groups' sums added by a fixed-order tree in LDS (`partial`, a float4 a thread); every
+// thread returns the total of its column slice.
+__device__ __forceinline__ float4 group_tree(float4 *partial, float4 acc, int width, int groups) {
+  const int g = threadIdx.x / width;
+  partial[threadIdx.x] = acc;
+  __syncthreads();
+  int stride = 1;
+  while (2 * stride < groups) stride *= 2;           // half the groups, rounded up to a power of two
+  for (; stride > 0 && groups > 1; stride /= 2) {
+    if (g < stride && g + stride < groups) {
+      float4 o = partial[threadIdx.x + stride * width];
+      float4 s = partial[threadIdx.x];
+      partial[threadIdx.x] = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
+    }
+    __syncthreads();
+  }
+  return partial[threadIdx.x % width];
 }
 // Sum over rows [t0, end) of probs[t] * values[t, :] in the vector layout; the threads of group 0
 // (threadIdx.x < D/4) return their float4 of it. `haveFirst`: `first` holds this thread's first
@@ -1578,19 +1596,7 @@ __device__ __forceinline__ float4 values_reduce(const float *values, int D, cons
     load_value_batch<NT>(vb, values, D, base, end);
     consume(vb, base);
   }
-  partial[threadIdx.x] = acc;
-  __syncthreads();
-  int stride = 1;
-  while (2 * stride < groups) stride *= 2;           // half the groups, rounded up to a power of two
-  for (; stride > 0 && groups > 1; stride /= 2) {
-    if (g < stride && g + stride < groups) {
-      float4 o = partial[threadIdx.x + stride * width];
-      float4 s = partial[threadIdx.x];
-      partial[threadIdx.x] = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
-    }
-    __syncthreads();
-  }
-  return partial[threadIdx.x % width];
+  return group_tree(partial, acc, width, groups);
 }
 // `haveFirst`: `first` holds this thread's first batch (vector layout, end > 0). `p` is the
 // position (a.position[0]), loaded by the caller.
@@ -1621,6 +1627,45 @@ template <bool NT> __device__ void attention_values_body(const ValuesArgs &a, in
 }
 CKL_ENTRY_ATTR(attention_values, ValuesArgs, attention_values_body<false>, kValuesBlock, )
 CKL_ENTRY_ATTR(attention_values_nt, ValuesArgs, attention_values_body<true>, kValuesBlock, )
+
+// attention_values for few long rows (python/ckl/library.py, _values): `slices` workgroups per
+// (b, h), each the weighted sum of its share of the rows at the current position; the last to arrive
+// adds the slices' sums (row groups take every groups-th slice in order, then the tree above) and
+// writes dst. Bound by the value stream: one workgroup alone reads ~50 GB/s whatever its depth.
+// 16 rows of 8001 x 128: 90.6 us one workgroup a row, 18.8 us in 16 slices (3.5 TB/s, the launch's
+// ramp and the combine's coherent round trips ~6 us of it).
+template <bool NT> __device__ void attention_values_split_body(const ValuesSplitArgs &a, int block) {
+  __shared__ float4 sums[kValuesBlock];
+  const long bh = block / a.slices;
+  const int slice = block % a.slices;
+  if (bh >= long(a.B) * a.A) return;
+  const int p = load_position(a.position);
+  const int end = p < 0 ? 0 : min(p + 1, a.T);
+  const int width = a.D / 4, groups = int(blockDim.x) / width;
+  const int g = threadIdx.x / width, part = threadIdx.x % width;
+  const int rows = (end + a.slices - 1) / a.slices;
+  const int t0 = min(slice * rows, end), t1 = min(t0 + rows, end);
+  const float *values = a.vc + (long(a.layer) * a.B * a.A + bh) * long(a.T) * a.D;
+  ValueBatch none;
+  const float4 sum = values_reduce<NT>(values, a.D, a.probs + bh * a.T, t0, t1, none, false);
+  float *planes = a.partials + bh * a.slices * a.D;
+  if (g == 0) {
+    const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+    partial_store_columns<4>(planes + long(slice) * a.D + 4 * part, v, true);
+  }
+  if (!split_arrive(reinterpret_cast<unsigned *>(a.workspace) + bh, a.slices)) return;
+  float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (g < groups)
+    for (int s = g; s < a.slices; s += groups) {
+      const FinishValue<2> lo = partial_load_n<2>(planes + long(s) * a.D + 4 * part);
+      const FinishValue<2> hi = partial_load_n<2>(planes + long(s) * a.D + 4 * part + 2);
+      total.x += lo.v[0]; total.y += lo.v[1]; total.z += hi.v[0]; total.w += hi.v[1];
+    }
+  const float4 all = group_tree(sums, total, width, groups);
+  if (g == 0) reinterpret_cast<float4 *>(a.dst + bh * a.D)[part] = all;
+}
+CKL_ENTRY_ATTR(attention_values_split, ValuesSplitArgs, attention_values_split_body<false>, kValuesBlock, )
+CKL_ENTRY_ATTR(attention_values_split_nt, ValuesSplitArgs, attention_values_split_body<true>, kValuesBlock, )
 
 // softmax -> attention_values as one launch of attention_values's geometry (one workgroup per
 // (b, h), blockDim >= rowThreads, checked by the executor): lanes [0, rowThreads) compute the

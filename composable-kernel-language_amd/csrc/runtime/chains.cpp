@@ -942,6 +942,10 @@ bool streams(const Launch &l) {
     const ValuesArgs a = block<ValuesArgs>(l);
     return int64_t(a.B) * a.A * a.T * a.D * 4 >= kStreamBytes;
   }
+  if (name == "ckl_attention_values_split" && l.arguments.size() == sizeof(ValuesSplitArgs)) {
+    const ValuesSplitArgs a = block<ValuesSplitArgs>(l);
+    return int64_t(a.B) * a.A * a.T * a.D * 4 >= kStreamBytes;
+  }
   return false;
 }
 

@@ -255,8 +255,37 @@ def _softmax(shapes, consts, ext):
     b, a, t = shapes[0]
     if not (ext[0] >= b and ext[1:] == (a, 1)):
         return None
-    row_threads = 64 if t <= 512 else 256           # one wave per row, or the whole workgroup
-    return Launch(_cdiv(b * a, BLOCK // row_threads), (b, a, t, row_threads))
+    # One wave per row, or a workgroup: 256 threads, or 1024 on rows so long that the values of few
+    # rows are always split, so that no chain wants softmax and values in one workgroup (256 threads
+    # stream a row of more than 2048 three times: 16 rows of 8001 19.7 -> 5.4 us).
+    row_threads = 64 if t <= 512 else 1024 if t > SOFTMAX_WIDE_ROW and b * a <= VALUES_SPLIT_HEADS else 256
+    block = max(BLOCK, row_threads)
+    return Launch(_cdiv(b * a, block // row_threads), (b, a, t, row_threads), block=block)
+
+
+# Long contexts of few requests: a workgroup per (b, h) row leaves most of the chip idle, and one
+# workgroup streams only ~50 GB/s. The rows are then cut into slices (ckl_attention_values_split),
+# and the chains that need a whole row in one workgroup are left for their parts (rope -> append_kv,
+# scores, softmax, values): 9 us more of launches, which at least 512 KB of values a row pay for, and
+# 16 KB more of them for every (b, h) row (attention layer, chain -> split, graph/ordinary us: 16 rows
+# of 8192 x 128 187/178 -> 61/83, of 1040 x 128 46/72 -> 43/66, of 512 x 128 31/60 -> 38/61; 64 rows of
+# 4096 x 128 113/134 -> 81/100, of 1040 x 128 49/75 -> 50/70; 128 rows of 2048 x 128 74/106 -> 80/101).
+# About VALUES_SPLIT_GROUPS workgroups, but 16 slices or one per 128 KB (8 rows of 8192 x 64: 16 slices
+# 34.5, 64 37.4, 128 44.3 us: the last workgroup adds them; 4 rows of 8192 x 128: 16 41.0, 32 38.4).
+VALUES_SPLIT_HEADS = 64
+VALUES_SPLIT_BYTES = 1 << 19
+VALUES_SPLIT_HEAD_BYTES = 1 << 14
+VALUES_SPLIT_GROUPS = 512
+SOFTMAX_WIDE_ROW = 6144
+
+
+def _values_slices(heads: int, t: int, d: int) -> int:
+    """Slices per (b, h) row of the values' sum (1: one workgroup a row)."""
+    if heads > VALUES_SPLIT_HEADS or d % 4 or d > 256:
+        return 1
+    if t <= SOFTMAX_WIDE_ROW and 4 * t * d < max(VALUES_SPLIT_BYTES, heads * VALUES_SPLIT_HEAD_BYTES):
+        return 1
+    return max(1, min(_cdiv(VALUES_SPLIT_GROUPS, heads), max(16, 4 * t * d >> 17), t // 64))
 
 
 def _values(shapes, consts, ext):
@@ -270,6 +299,10 @@ def _values(shapes, consts, ext):
     block = 64
     while block < VALUES_BLOCK and (block // width) * 8 < t:
         block *= 2
+    slices = _values_slices(b * a, t, d)
+    if slices > 1:
+        return Launch(b * a * slices, (l, b, a, t, d, layer, slices), block=256, entry="ckl_attention_values_split",
+                      workspace=_cdiv(4 * b * a, 256) * 256, partials=4 * b * a * slices * d)
     return Launch(b * a, (l, b, a, t, d, layer), block=block)
 
 
