@@ -37,6 +37,13 @@ std::string unsignedType(const Type &t) {
   }
 }
 
+size_t elementBytes(const Type &memref) {
+  switch (memref.element) {
+  case Type::F64: case Type::I64: case Type::Index: return 8;
+  default: return 4;
+  }
+}
+
 std::string literal(const Attr &a) {
   char buf[64];
   if (a.kind == Attr::Float) {
@@ -73,8 +80,81 @@ public:
       std::string n = bind(entry->args[k].get());
       out << "  " << cType(entry->args[k]->type) << " " << n << " = args.a" << k << ";\n";
     }
-    for (auto &op : entry->ops) statement(*op, 1);
+    const Attr *elements = function.attr("ckl.hip.elements_per_thread");
+    if (elements && elements->i > 1) elementwise(*entry, elements->i);
+    else for (auto &op : entry->ops) statement(*op, 1);
     out << "}\n\n";
+  }
+
+  // An elementwise kernel (csrc/core/analysis.cpp, vectorizeElementwise): this thread's `n`
+  // consecutive elements with one vector load per buffer read, the body once per element, and one
+  // vector store per buffer written; the vector's last, incomplete group element by element. Buffers
+  // may start at any element, so the vectors are aligned as their elements. Bound by memory: stores of
+  // a buffer that no cache holds bypass them (of 2^26 floats, 72 us against 87 us with plain stores).
+  void elementwise(const Block &entry, int64_t n) {
+    constexpr int64_t streamBytes = int64_t(8) << 20;
+    const Op *guard = nullptr;
+    const Value *index = nullptr;
+    for (auto &op : entry.ops) {
+      if (op->name == "scf.if") guard = op.get();
+      else if (op->name == "ckl.global_id") index = op->result();
+      else if (op->name == "arith.constant") statement(*op, 1);
+    }
+    if (!guard || !index) throw CompileError("device code generation: not an elementwise kernel");
+    const Block &body = *guard->regions[0]->blocks[0];
+    std::vector<const Value *> read, written;
+    auto place = [](std::vector<const Value *> &set, const Value *v) {
+      for (size_t k = 0; k < set.size(); ++k) if (set[k] == v) return k;
+      set.push_back(v);
+      return set.size() - 1;
+    };
+    for (auto &op : body.ops) {
+      if (op->name == "ckl.load_element") place(read, op->operands[0]);
+      if (op->name == "ckl.store_element") place(written, op->operands[1]);
+    }
+    int64_t count = 0;
+    for (const auto *set : {&read, &written}) for (const Value *v : *set) count = v->type.shape.at(0);
+    auto vectorType = [&](const Value *v, const std::string &name) {
+      const std::string t = cType(Type::scalar(v->type.element));
+      out << "  typedef " << t << " " << name << " __attribute__((ext_vector_type(" << n << "), aligned(sizeof(" << t << "))));\n";
+    };
+    for (size_t k = 0; k < read.size(); ++k) vectorType(read[k], "load" + std::to_string(k) + "_t");
+    for (size_t k = 0; k < written.size(); ++k) vectorType(written[k], "store" + std::to_string(k) + "_t");
+    out << "  const long long first = ((long long)blockIdx.x * (long long)blockDim.x + (long long)threadIdx.x) * " << n << "LL;\n";
+    out << "  if (first + " << n << "LL <= " << count << "LL) {\n";
+    for (size_t k = 0; k < read.size(); ++k)
+      out << "    const load" << k << "_t l" << k << " = *(const load" << k << "_t *)(" << ref(read[k]) << " + first);\n";
+    for (size_t k = 0; k < written.size(); ++k) out << "    store" << k << "_t s" << k << ";\n";
+    for (int64_t e = 0; e < n; ++e) {
+      out << "    {\n      const long long " << bind(index) << " = first + " << e << "LL;\n";
+      comparisons(entry);
+      for (auto &op : body.ops) {
+        if (op->name == "ckl.load_element")
+          out << "      const " << cType(op->results[0]->type) << " " << bind(op->results[0].get()) << " = l"
+              << place(read, op->operands[0]) << "[" << e << "];\n";
+        else if (op->name == "ckl.store_element")
+          out << "      s" << place(written, op->operands[1]) << "[" << e << "] = " << ref(op->operands[0]) << ";\n";
+        else if (op->name != "scf.yield") statement(*op, 3);
+      }
+      out << "    }\n";
+    }
+    for (size_t k = 0; k < written.size(); ++k) {
+      const std::string type = "store" + std::to_string(k) + "_t", at = "(" + type + " *)(" + ref(written[k]) + " + first)";
+      if (count * int64_t(elementBytes(written[k]->type)) >= streamBytes)
+        out << "    __builtin_nontemporal_store(s" << k << ", " << at << ");\n";
+      else out << "    *" << at << " = s" << k << ";\n";
+    }
+    const std::string i = bind(index);
+    out << "  } else {\n    for (long long " << i << " = first; " << i << " < " << count << "LL; ++" << i << ") {\n";
+    comparisons(entry);
+    for (auto &op : body.ops)
+      if (op->name != "scf.yield") statement(*op, 3);
+    out << "    }\n  }\n";
+  }
+  // The comparisons ahead of the guard, of the index now bound (the body may use them).
+  void comparisons(const Block &entry) {
+    for (auto &op : entry.ops)
+      if (op->name == "arith.cmpi") statement(*op, 3);
   }
 
 private:
