@@ -131,6 +131,12 @@ struct CKL_ALIGN RopeAttentionChainArgs {
   PartialSource qsrc, ksrc, v;
 };
 
+// rope(q), rope(k) -> append_kv -> attention_scores in the scores' geometry (values cut into slices).
+struct CKL_ALIGN RopeScoresChainArgs {
+  RopeArgs q; RopeArgs k; AppendArgs append; ScoresArgs scores;
+  PartialSource qsrc, ksrc, v;
+};
+
 // Whether attention rows of D floats take the scores' padded vector layout (library.hip,
 // attention_scores): a multiple of 4 up to 256 that no exact layout covers.
 constexpr bool scoresPadded(int D) {

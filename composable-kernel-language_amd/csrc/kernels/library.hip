@@ -1941,6 +1941,101 @@ CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores__softmax__attention_val
 CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores__softmax__attention_values_padded_nt, RopeAttentionChainArgs,
                  (rope_attention_rows<true, 0>), kValuesBlock, )
 
+// rope(q), rope(k) -> append_kv -> attention_scores in one launch of attention_scores' geometry, for
+// contexts whose values are cut into slices: every workgroup of (b, h) rotates the head's q into LDS
+// (the first writes it), the one whose chunk holds the position appends k and v and takes that key row
+// from LDS. A thread's rotation operands are requested before the wave's first key rows, as in the
+// chain above. D is a multiple of 4 up to 256 (the vector layouts), so R <= 128 threads rotate a pair
+// each. A position outside [0, T) does what the separate launches do. Bound by the key stream and its
+// launch; 16 rows of 8001 x 128, an attention layer: 78.4 us with rope -> append_kv launched before the
+// scores, 70.8 us with both in one launch.
+template <bool NT, int K> __device__ void rope_scores_rows(const RopeScoresChainArgs &a, int block) {
+  __shared__ float4 rotated[2][64];
+  float *qrow = reinterpret_cast<float *>(rotated[0]), *krow = reinterpret_cast<float *>(rotated[1]);
+  constexpr int P = KeyLayout<K>::P;
+  const RopeArgs &q = a.q, &k = a.k;
+  const AppendArgs &ap = a.append;
+  const ScoresArgs &sc = a.scores;
+  const int chunks = (sc.T + kBlock - 1) / kBlock;
+  const long bh = block / chunks;
+  if (bh >= long(sc.B) * sc.A) return;
+  const int t0 = block % chunks * kBlock;
+  const int p = load_position(q.position);
+  const int end = min(p + 1, sc.T);
+  if (p < 0 || t0 >= end) return;
+  const bool inRange = p < sc.T;
+  const int tEnd = min(t0 + kBlock, end);
+  const bool owner = inRange && tEnd == end;           // the chunk that holds the position
+  const KeyLayout<K> layout(sc.D);
+  const float *keys = sc.kc + (long(sc.layer) * sc.B * sc.A + bh) * long(sc.T) * sc.D;
+  const int pair = threadIdx.x;
+  const bool rotates = inRange && pair < q.R;
+  const long pairIndex = bh * (2L * q.R) + 2 * pair;
+  const bool request = a.qsrc.parts <= kRopeRequest && a.ksrc.parts <= kRopeRequest && a.v.parts <= kRopeRequest;
+  float2 qPlanes[kRopeRequest], kPlanes[kRopeRequest], vPlanes[kRopeRequest], table = make_float2(0.f, 0.f);
+  if (rotates) {
+    table = *reinterpret_cast<const float2 *>(q.table + long(p) * q.R * 2 + 2 * pair);
+    if (request) {
+      request_pair(a.qsrc, q.src, pairIndex, qPlanes);
+      if (owner) {
+        request_pair(a.ksrc, k.src, pairIndex, kPlanes);
+        request_pair(a.v, ap.v, pairIndex, vPlanes);
+      }
+    }
+  }
+  // The wave's 64 rows; the appended row comes from LDS and is never read from the cache here.
+  const int w0 = t0 + int(threadIdx.x >> 6) * 64, w1 = min(min(w0 + 64, tEnd), owner ? end - 1 : end);
+  KeyBatch first;
+  if (w0 < w1) load_key_batch<NT, K>(first, keys + long(w0) * sc.D, sc.D, layout, 0, w1 - w0);
+  if (rotates) {
+    const float2 qr = rotate(request ? sum_pair(a.qsrc, qPlanes) : source2(a.qsrc, q.src, pairIndex), table);
+    *reinterpret_cast<float2 *>(qrow + 2 * pair) = qr;
+    if (t0 == 0) *reinterpret_cast<float2 *>(q.dst + pairIndex) = qr;
+    if (owner) {
+      const long row = ((long(ap.layer) * ap.B * ap.A + bh) * ap.T + p) * ap.D + 2 * pair;
+      const float2 kr = rotate(request ? sum_pair(a.ksrc, kPlanes) : source2(a.ksrc, k.src, pairIndex), table);
+      *reinterpret_cast<float2 *>(krow + 2 * pair) = kr;
+      if (k.dst) *reinterpret_cast<float2 *>(k.dst + pairIndex) = kr;
+      *reinterpret_cast<float2 *>(ap.kc + row) = kr;
+      *reinterpret_cast<float2 *>(ap.vc + row) = request ? sum_pair(a.v, vPlanes) : source2(a.v, ap.v, pairIndex);
+    }
+  }
+  __syncthreads();
+  float *scores = sc.scores + bh * sc.T;
+  float4 qv[P];
+  layout.loadQuery(qv, inRange ? qrow : sc.q + bh * sc.D);
+  auto score = [&](const KeyBatch &kb, int base) {
+#pragma unroll
+    for (int u = 0; u < layout.U; ++u) {
+      const float v = group_sum(layout.dot(qv, kb.kv + u * P), layout.G) * sc.scale;
+      const int t = base + u * layout.rowsPerLoad + layout.sub;
+      if (layout.part == 0 && t < w1) scores[t] = v;
+    }
+  };
+  if (w0 < w1) score(first, w0);
+  for (int base = w0 + layout.rowsPerBatch(); base < w1; base += layout.rowsPerBatch()) {
+    KeyBatch kb;
+    load_key_batch<NT, K>(kb, keys + long(w0) * sc.D, sc.D, layout, base - w0, w1 - w0);
+    score(kb, base);
+  }
+  if (owner && threadIdx.x < 64) {
+    float4 kv[P];
+    layout.loadQuery(kv, krow);
+    const float v = group_sum(layout.dot(qv, kv), layout.G) * sc.scale;
+    if (threadIdx.x == 0) scores[p] = v;
+  }
+}
+template <bool NT> __device__ void rope_scores_body(const RopeScoresChainArgs &a, int block) {
+  switch (score_layout(a.scores.D)) {
+    case 0: rope_scores_rows<NT, 0>(a, block); break;
+    case 1: rope_scores_rows<NT, 1>(a, block); break;
+    case 2: rope_scores_rows<NT, 2>(a, block); break;
+    default: rope_scores_rows<NT, 4>(a, block); break;
+  }
+}
+CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores, RopeScoresChainArgs, rope_scores_body<false>, kBlock, )
+CKL_SINGLE_ENTRY(rope__rope__append_kv__attention_scores_nt, RopeScoresChainArgs, rope_scores_body<true>, kBlock, )
+
 // ------------------------------------------------------------------ pointwise
 // add: dst = x + y; multiply: dst = x * y; silu: dst = v / (1 + exp(-v)) (workloads.py:145-167).
 

@@ -5,7 +5,7 @@
 // entry points (csrc/kernels/library.hip) that run several dependent dispatches row by row in one
 // grid: rms_stats -> rms_apply, add -> rms_stats -> rms_apply, embedding -> rms_stats ->
 // rms_apply, silu -> multiply, rope(q), rope(k) -> append_kv -> attention_scores -> softmax ->
-// attention_values (or the rope part alone, attention_scores -> softmax -> attention_values, or
+// attention_values (or the rope part alone or with attention_scores, scores -> softmax -> values, or
 // softmax -> attention_values), greedy -> advance, and for row-parallel linears whose workgroups
 // hold whole rows, linear -> add -> rms_stats -> rms_apply and linear, linear -> silu -> multiply
 // (both as one launch for single-wave linears). add alone is a chain of one, so that it can read a
@@ -357,6 +357,42 @@ const char *ropeAttentionChain(const Members &m, const Internal &internal, Launc
   return nullptr;
 }
 
+// rope(q), rope(k) -> append_kv -> attention_scores whose values are cut into slices: the scores'
+// workgroups of one (b, h) all read its q and one of them writes the rotated rows, so nothing written
+// may overlap anything else.
+const char *ropeScoresChain(const Members &m, const Internal &internal, Launch &out) {
+  RopeScoresChainArgs c{block<RopeArgs>(*m[0]), block<RopeArgs>(*m[1]), block<AppendArgs>(*m[2]), block<ScoresArgs>(*m[3]),
+                        {}, {}, {}};
+  const RopeArgs &q = c.q, &k = c.k;
+  const AppendArgs &ap = c.append;
+  const ScoresArgs &sc = c.scores;
+  if (q.table != k.table || q.position != k.position || q.position != ap.position || q.position != sc.position ||
+      q.B != k.B || q.A != k.A || q.R != k.R || q.T != k.T)
+    return "the two ropes disagree on table, position or shape";
+  if (ap.k != k.dst || ap.B != q.B || ap.A != q.A || ap.D != 2 * q.R || ap.T != q.T || ap.layer < 0 || ap.L <= ap.layer)
+    return "append_kv does not take the rotated k";
+  if (sc.q != q.dst || sc.kc != ap.kc || sc.layer != ap.layer || sc.L != ap.L || sc.B != q.B || sc.A != q.A ||
+      sc.T != q.T || sc.D != ap.D)
+    return "the scores do not read the rotated q and the appended cache";
+  if (q.B <= 0 || q.A <= 0 || q.R <= 0 || q.T <= 0) return "empty rope";
+  if (ap.D % 4 || ap.D > 256) return "the head size has no vector layout";
+  const uint64_t bh = uint64_t(q.B) * uint64_t(q.A), head = 4 * bh * uint64_t(ap.D);
+  const uint64_t cache = bh * uint64_t(ap.T) * uint64_t(ap.D);
+  if (internal(1, k.dst)) c.k.dst = nullptr;
+  std::vector<Range> written{slab(q.dst, head, true), slab(sc.scores, 4 * bh * uint64_t(q.T), true),
+                             slab(ap.kc + int64_t(ap.layer) * int64_t(cache), 4 * cache, true),
+                             slab(ap.vc + int64_t(ap.layer) * int64_t(cache), 4 * cache, true)};
+  if (c.k.dst) written.push_back(slab(k.dst, head, true));
+  const std::vector<Range> read{whole(q.src, head), whole(k.src, head), whole(ap.v, head),
+                                whole(q.table, 8ull * uint64_t(q.T) * uint64_t(q.R)), whole(q.position, 4)};
+  if (!writesDisjoint(written, read)) return kOverlap;
+  out.grid[0] = m[3]->grid[0];
+  out.block[0] = m[3]->block[0];
+  out.shared = 0;
+  setArguments(out, c);
+  return nullptr;
+}
+
 // Row-parallel linear whose workgroup holds a whole output row (one tile, one slice) -> add ->
 // rms_stats -> rms_apply: one workgroup per batch row.
 const char *linearAddRmsChain(const Members &m, const Internal &internal, Launch &out) {
@@ -624,6 +660,30 @@ std::vector<size_t> matchRopeAttention(const Plan &plan, size_t head, const Succ
   return roles;
 }
 
+// The rope chain's three roles, then attention_scores taking the rotated q and reading the appended
+// cache, where a softmax and values in slices follow.
+std::vector<size_t> matchRopeScores(const Plan &plan, size_t head, const Successors &successors,
+                                    const std::vector<bool> &taken) {
+  std::vector<size_t> roles = matchRopeAppend(plan, head, successors, taken);
+  if (roles.size() != 3) return {};
+  const void *rotatedQ = block<RopeArgs>(plan.nodes[roles[0]].launch).dst;
+  auto next = [&](size_t from, const char *name) {
+    size_t found = plan.nodes.size();
+    for (size_t s : successors[from]) {
+      const Launch &l = plan.nodes[s].launch;
+      if (!taken[s] && l.name == name && singleGrid(l) && s < found) found = s;
+    }
+    return found;
+  };
+  const size_t n = plan.nodes.size();
+  const size_t scores = next(roles[2], "ckl_attention_scores");
+  if (scores == n || block<ScoresArgs>(plan.nodes[scores].launch).q != rotatedQ) return {};
+  const size_t softmax = next(scores, "ckl_softmax");
+  if (softmax == n || next(softmax, "ckl_attention_values_split") == n) return {};
+  roles.push_back(scores);
+  return roles;
+}
+
 std::vector<size_t> matchLinearSilu(const Plan &plan, size_t head, const Successors &successors,
                                     const std::vector<bool> &taken);
 
@@ -731,6 +791,11 @@ const std::vector<Rule> &rules() {
        {{0, offsetof(RopeArgs, src), offsetof(RopeAttentionChainArgs, qsrc)},
         {1, offsetof(RopeArgs, src), offsetof(RopeAttentionChainArgs, ksrc)},
         {2, offsetof(AppendArgs, v), offsetof(RopeAttentionChainArgs, v)}}},
+      {{"ckl_rope", "ckl_rope", "ckl_append_kv", "ckl_attention_scores"}, "ckl_rope__rope__append_kv__attention_scores",
+       ropeScoresChain, matchRopeScores,
+       {{0, offsetof(RopeArgs, src), offsetof(RopeScoresChainArgs, qsrc)},
+        {1, offsetof(RopeArgs, src), offsetof(RopeScoresChainArgs, ksrc)},
+        {2, offsetof(AppendArgs, v), offsetof(RopeScoresChainArgs, v)}}},
       {{"ckl_linear_rowvec", "ckl_add", "ckl_rms_stats", "ckl_rms_apply", "ckl_linear_rowvec", "ckl_linear_rowvec",
         "ckl_silu", "ckl_multiply"},
        "ckl_linear_rowvec__add__rms_stats__rms_apply__linear_rowvec__linear_rowvec__silu__multiply",

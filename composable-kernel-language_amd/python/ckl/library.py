@@ -265,8 +265,9 @@ def _softmax(shapes, consts, ext):
 
 # Long contexts of few requests: a workgroup per (b, h) row leaves most of the chip idle, and one
 # workgroup streams only ~50 GB/s. The rows are then cut into slices (ckl_attention_values_split),
-# and the chains that need a whole row in one workgroup are left for their parts (rope -> append_kv,
-# scores, softmax, values): 9 us more of launches, which at least 512 KB of values a row pay for, and
+# and the chain that needs a whole row in one workgroup is left for its parts (rope -> append_kv ->
+# scores, softmax, values): launches of about 6 us more (9 us for the figures here, rope -> append_kv
+# still apart), which at least 512 KB of values a row pay for, and
 # 16 KB more of them for every (b, h) row (attention layer, chain -> split, graph/ordinary us: 16 rows
 # of 8192 x 128 187/178 -> 61/83, of 1040 x 128 46/72 -> 43/66, of 512 x 128 31/60 -> 38/61; 64 rows of
 # 4096 x 128 113/134 -> 81/100, of 1040 x 128 49/75 -> 50/70; 128 rows of 2048 x 128 74/106 -> 80/101).
