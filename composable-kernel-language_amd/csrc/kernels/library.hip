@@ -1632,8 +1632,8 @@ CKL_ENTRY_ATTR(attention_values_nt, ValuesArgs, attention_values_body<true>, kVa
 // (b, h), each the weighted sum of its share of the rows at the current position; the last to arrive
 // adds the slices' sums (row groups take every groups-th slice in order, then the tree above) and
 // writes dst. Bound by the value stream: one workgroup alone reads ~50 GB/s whatever its depth.
-// 16 rows of 8001 x 128: 90.6 us one workgroup a row, 18.8 us in 16 slices (3.5 TB/s, the launch's
-// ramp and the combine's coherent round trips ~6 us of it).
+// 16 rows of 8001 x 128: 90.6 us one workgroup a row, 18.8 us in 32 slices of 256 threads (3.5 TB/s,
+// the launch's ramp and the combine's coherent round trips ~6 us of it), 3 us less in 16 of 512.
 template <bool NT> __device__ void attention_values_split_body(const ValuesSplitArgs &a, int block) {
   __shared__ float4 sums[kValuesBlock];
   const long bh = block / a.slices;

@@ -273,10 +273,13 @@ def _softmax(shapes, consts, ext):
 # 4096 x 128 113/134 -> 81/100, of 1040 x 128 49/75 -> 50/70; 128 rows of 2048 x 128 74/106 -> 80/101).
 # About VALUES_SPLIT_GROUPS workgroups, but 16 slices or one per 128 KB (8 rows of 8192 x 64: 16 slices
 # 34.5, 64 37.4, 128 44.3 us: the last workgroup adds them; 4 rows of 8192 x 128: 16 41.0, 32 38.4).
+# One workgroup of 512 threads per compute unit (attention layer, us, 16 rows of 8192 x 128 / 64 rows of
+# 4096 x 64: 512 of 256 threads 72.1 / 72.3, 512 of 512 71.5 / 72.3, 384 of 512 68.7 / 72.7, 256 of 512
+# 67.4 / 70.2, 192 of 512 68.2 / 71.4; 256 of 256 69.8 / 72.5).
 VALUES_SPLIT_HEADS = 64
 VALUES_SPLIT_BYTES = 1 << 19
 VALUES_SPLIT_HEAD_BYTES = 1 << 14
-VALUES_SPLIT_GROUPS = 512
+VALUES_SPLIT_GROUPS = 256
 SOFTMAX_WIDE_ROW = 6144
 
 
@@ -302,7 +305,7 @@ def _values(shapes, consts, ext):
         block *= 2
     slices = _values_slices(b * a, t, d)
     if slices > 1:
-        return Launch(b * a * slices, (l, b, a, t, d, layer, slices), block=256, entry="ckl_attention_values_split",
+        return Launch(b * a * slices, (l, b, a, t, d, layer, slices), block=VALUES_BLOCK, entry="ckl_attention_values_split",
                       workspace=_cdiv(4 * b * a, 256) * 256, partials=4 * b * a * slices * d)
     return Launch(b * a, (l, b, a, t, d, layer), block=block)
 
