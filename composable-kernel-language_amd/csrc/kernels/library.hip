@@ -1564,7 +1564,7 @@ __device__ __forceinline__ float4 group_tree(float4 *partial, float4 acc, int wi
 }
 // Sum over rows [t0, end) of probs[t] * values[t, :] in the vector layout; the threads of group 0
 // (threadIdx.x < D/4) return their float4 of it. `haveFirst`: `first` holds this thread's first
-// batch (t0 = 0, end > 0). The groups' sums are added by a fixed-order tree in LDS.
+// batch (t0 < end). The groups' sums are added by a fixed-order tree in LDS.
 template <bool NT>
 __device__ __forceinline__ float4 values_reduce(const float *values, int D, const float *probs, int t0, int end,
                                                 const ValueBatch &first, bool haveFirst) {
@@ -1588,8 +1588,8 @@ __device__ __forceinline__ float4 values_reduce(const float *values, int D, cons
   };
   int base = t0;
   if (haveFirst) {
-    consume(first, 0);
-    base = step;
+    consume(first, t0);
+    base += step;
   }
   for (; base < end; base += step) {
     ValueBatch vb;
@@ -1634,20 +1634,11 @@ CKL_ENTRY_ATTR(attention_values_nt, ValuesArgs, attention_values_body<true>, kVa
 // writes dst. Bound by the value stream: one workgroup alone reads ~50 GB/s whatever its depth.
 // 16 rows of 8001 x 128: 90.6 us one workgroup a row, 18.8 us in 32 slices of 256 threads (3.5 TB/s,
 // the launch's ramp and the combine's coherent round trips ~6 us of it), 3 us less in 16 of 512.
-template <bool NT> __device__ void attention_values_split_body(const ValuesSplitArgs &a, int block) {
+// The slice's sum goes to its plane; the last slice of the row adds them.
+__device__ __forceinline__ void values_split_finish(const ValuesSplitArgs &a, long bh, int slice, float4 sum) {
   __shared__ float4 sums[kValuesBlock];
-  const long bh = block / a.slices;
-  const int slice = block % a.slices;
-  if (bh >= long(a.B) * a.A) return;
-  const int p = load_position(a.position);
-  const int end = p < 0 ? 0 : min(p + 1, a.T);
   const int width = a.D / 4, groups = int(blockDim.x) / width;
   const int g = threadIdx.x / width, part = threadIdx.x % width;
-  const int rows = (end + a.slices - 1) / a.slices;
-  const int t0 = min(slice * rows, end), t1 = min(t0 + rows, end);
-  const float *values = a.vc + (long(a.layer) * a.B * a.A + bh) * long(a.T) * a.D;
-  ValueBatch none;
-  const float4 sum = values_reduce<NT>(values, a.D, a.probs + bh * a.T, t0, t1, none, false);
   float *planes = a.partials + bh * a.slices * a.D;
   if (g == 0) {
     const float v[4] = {sum.x, sum.y, sum.z, sum.w};
@@ -1663,6 +1654,25 @@ template <bool NT> __device__ void attention_values_split_body(const ValuesSplit
     }
   const float4 all = group_tree(sums, total, width, groups);
   if (g == 0) reinterpret_cast<float4 *>(a.dst + bh * a.D)[part] = all;
+}
+// Rows [t0, t1) of `slice` when the row ends at `end`.
+__device__ __forceinline__ void values_slice(const ValuesSplitArgs &a, int slice, int end, int &t0, int &t1) {
+  const int rows = (end + a.slices - 1) / a.slices;
+  t0 = min(slice * rows, end);
+  t1 = min(t0 + rows, end);
+}
+template <bool NT> __device__ void attention_values_split_body(const ValuesSplitArgs &a, int block) {
+  const long bh = block / a.slices;
+  const int slice = block % a.slices;
+  if (bh >= long(a.B) * a.A) return;
+  const int p = load_position(a.position);
+  const int end = p < 0 ? 0 : min(p + 1, a.T);
+  int t0, t1;
+  values_slice(a, slice, end, t0, t1);
+  const float *values = a.vc + (long(a.layer) * a.B * a.A + bh) * long(a.T) * a.D;
+  ValueBatch none;
+  const float4 sum = values_reduce<NT>(values, a.D, a.probs + bh * a.T, t0, t1, none, false);
+  values_split_finish(a, bh, slice, sum);
 }
 CKL_ENTRY_ATTR(attention_values_split, ValuesSplitArgs, attention_values_split_body<false>, kValuesBlock, )
 CKL_ENTRY_ATTR(attention_values_split_nt, ValuesSplitArgs, attention_values_split_body<true>, kValuesBlock, )
@@ -1685,6 +1695,106 @@ template <bool NT> __device__ void softmax__attention_values_body(const SoftmaxV
 }
 CKL_ENTRY_ATTR(softmax__attention_values, SoftmaxValuesChainArgs, softmax__attention_values_body<false>, kValuesBlock, )
 CKL_ENTRY_ATTR(softmax__attention_values_nt, SoftmaxValuesChainArgs, softmax__attention_values_body<true>, kValuesBlock, )
+
+// softmax -> attention_values in slices as one launch of the latter's geometry: the workgroup of every
+// slice repeats the softmax of its whole row (T <= kChainSoftmaxRow, 512 threads) with the arithmetic of
+// softmax_row, for its own rows' weights in LDS; its first value rows are requested before that. A
+// softmax of rowThreads lanes is run by 256 of them, or as two lanes a thread where it has 1024: both
+// keep each lane's sums in element order and add the waves' in wave order. A row longer than the lanes'
+// registers is staged in LDS (`row`, T floats) by all threads. Probabilities are not written. 16 rows of
+// 8001 x 128, an attention layer: 67.8 us with softmax as a launch, 65.5 us here.
+template <int Lanes> __device__ __forceinline__ void slice_weights(const SoftmaxArgs &a, const float *s, int end, int t0, int t1,
+                                                                   float *row) {
+  __shared__ float maxima[16], sums[16];
+  const int rowThreads = a.rowThreads, step = rowThreads / Lanes;
+  const bool active = int(threadIdx.x) < step;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int waves = rowThreads / 64;
+  float v[Lanes][kSoftmaxPerLane];
+  const bool held = end <= rowThreads * kSoftmaxPerLane;
+  if (!held) {
+    const int threads = blockDim.x;
+    for (int base = threadIdx.x; base < end; base += threads * kSoftmaxPerLane) {
+      float x[kSoftmaxPerLane];
+#pragma unroll
+      for (int u = 0; u < kSoftmaxPerLane; ++u) x[u] = s[min(base + u * threads, end - 1)];
+#pragma unroll
+      for (int u = 0; u < kSoftmaxPerLane; ++u)
+        if (base + u * threads < end) row[base + u * threads] = x[u];
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int h = 0; h < Lanes; ++h)
+#pragma unroll
+      for (int u = 0; u < kSoftmaxPerLane; ++u) v[h][u] = s[min(int(threadIdx.x) + h * step + u * rowThreads, end - 1)];
+  }
+#pragma unroll
+  for (int h = 0; h < Lanes; ++h) {
+    const int local = threadIdx.x + h * step;
+    float m = -__builtin_inff();
+    if (held) {
+#pragma unroll
+      for (int u = 0; u < kSoftmaxPerLane; ++u) {
+        if (!active || local + u * rowThreads >= end) v[h][u] = -__builtin_inff();
+        m = fmaxf(m, v[h][u]);
+      }
+    } else if (active) {
+      for (int t = local; t < end; t += rowThreads) m = fmaxf(m, row[t]);
+    }
+    m = wave_max(m);
+    if (lane == 0 && active) maxima[wave + h * (step / 64)] = m;
+  }
+  __syncthreads();
+  float m = maxima[0];
+  for (int w = 1; w < waves; ++w) m = fmaxf(m, maxima[w]);
+#pragma unroll
+  for (int h = 0; h < Lanes; ++h) {
+    const int local = threadIdx.x + h * step;
+    float total = 0.f;
+    if (held) {
+#pragma unroll
+      for (int u = 0; u < kSoftmaxPerLane; ++u) {
+        const int t = local + u * rowThreads;
+        v[h][u] = t < end ? expf(v[h][u] - m) : 0.f;
+        total += v[h][u];
+      }
+    } else if (active) {
+      for (int t = local; t < end; t += rowThreads) total += expf(row[t] - m);
+    }
+    total = wave_sum(total);
+    if (lane == 0 && active) sums[wave + h * (step / 64)] = total;
+  }
+  __syncthreads();
+  float total = sums[0];
+  for (int w = 1; w < waves; ++w) total = total + sums[w];
+  for (int t = t0 + int(threadIdx.x); t < t1; t += int(blockDim.x)) row[t] = expf((held ? s[t] : row[t]) - m) / total;
+  __syncthreads();
+}
+template <bool NT> __device__ void softmax__attention_values_split_body(const SoftmaxSplitChainArgs &a, int block) {
+  extern __shared__ float row[];
+  const ValuesSplitArgs &v = a.values;
+  const long bh = block / v.slices;
+  const int slice = block % v.slices;
+  if (bh >= long(v.B) * v.A) return;
+  const int p = load_position(v.position);
+  const int end = p < 0 ? 0 : min(p + 1, v.T);
+  int t0, t1;
+  values_slice(v, slice, end, t0, t1);
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (t0 < t1) {
+    const float *values = v.vc + ((long(v.layer) * v.B * v.A + bh) * long(v.T) + t0) * v.D;
+    ValueBatch first;
+    load_value_batch<NT>(first, values, v.D, 0, t1 - t0);
+    const float *s = a.softmax.scores + bh * v.T;
+    if (a.softmax.rowThreads == 1024) slice_weights<2>(a.softmax, s, end, t0, t1, row);
+    else slice_weights<1>(a.softmax, s, end, t0, t1, row);
+    sum = values_reduce<NT>(values, v.D, row + t0, 0, t1 - t0, first, true);
+  }
+  values_split_finish(v, bh, slice, sum);
+}
+CKL_SINGLE_ENTRY(softmax__attention_values_split, SoftmaxSplitChainArgs, softmax__attention_values_split_body<false>, kValuesBlock, )
+CKL_SINGLE_ENTRY(softmax__attention_values_split_nt, SoftmaxSplitChainArgs, softmax__attention_values_split_body<true>, kValuesBlock, )
 
 // attention_scores -> softmax -> attention_values as one launch of attention_values's geometry
 // (one workgroup per (b, h)): the workgroup computes the row's scores into LDS (the waves stride

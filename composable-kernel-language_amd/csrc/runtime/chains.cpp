@@ -244,6 +244,32 @@ Range slab(const void *p, uint64_t bytes, bool written) {
   return {a, a + bytes, written, false, 0};
 }
 
+// softmax whose rows only values in slices read: every slice's workgroup reads its whole row of scores.
+const char *softmaxSplitChain(const Members &m, const Internal &internal, Launch &out) {
+  SoftmaxSplitChainArgs c{block<SoftmaxArgs>(*m[0]), block<ValuesSplitArgs>(*m[1])};
+  const SoftmaxArgs &x = c.softmax;
+  const ValuesSplitArgs &v = c.values;
+  const Launch &values = *m[1];
+  if (x.probs != v.probs || x.position != v.position || x.B != v.B || x.A != v.A || x.T != v.T)
+    return "attention_values does not consume softmax's rows";
+  if (x.B <= 0 || x.A <= 0 || x.T <= 0 || x.T > kChainSoftmaxRow || v.D <= 0 || v.layer < 0 || v.slices <= 0)
+    return "softmax row does not fit the chain";
+  if (x.rowThreads != 64 && x.rowThreads != 256 && x.rowThreads != 1024) return "softmax row of another width";
+  if (values.block[0] != 512 || values.grid[0] != unsigned(x.B) * unsigned(x.A) * unsigned(v.slices))
+    return "attention_values runs another grid";
+  if (!internal(0, x.probs)) return "other readers take the probabilities";
+  const uint64_t bh = uint64_t(x.B) * uint64_t(x.A), cache = bh * uint64_t(x.T) * uint64_t(v.D);
+  if (!writesDisjoint({slab(v.dst, 4 * bh * uint64_t(v.D), true)},
+                      {whole(x.scores, 4 * bh * uint64_t(x.T)), whole(x.position, 4),
+                       whole(v.vc + int64_t(v.layer) * int64_t(cache), 4 * cache)}))
+    return kOverlap;
+  out.grid[0] = values.grid[0];
+  out.block[0] = values.block[0];
+  out.shared = unsigned(4 * x.T);
+  setArguments(out, c);
+  return nullptr;
+}
+
 const char *attentionChain(const Members &m, const Internal &internal, Launch &out) {
   AttentionChainArgs c{block<ScoresArgs>(*m[0]), block<SoftmaxArgs>(*m[1]), block<ValuesArgs>(*m[2])};
   const ScoresArgs &sc = c.scores;
@@ -819,6 +845,7 @@ const std::vector<Rule> &rules() {
       {{"ckl_attention_scores", "ckl_softmax", "ckl_attention_values"}, "ckl_attention_scores__softmax__attention_values",
        attentionChain},
       {{"ckl_softmax", "ckl_attention_values"}, "ckl_softmax__attention_values", softmaxValuesChain},
+      {{"ckl_softmax", "ckl_attention_values_split"}, "ckl_softmax__attention_values_split", softmaxSplitChain},
       {{"ckl_linear_rowvec", "ckl_greedy", "ckl_advance"}, "ckl_linear_rowvec__greedy__advance",
        linearGreedyAdvanceChain},
       {{"ckl_greedy", "ckl_advance"}, "ckl_greedy__advance", greedyAdvanceChain},

@@ -1,7 +1,7 @@
-"""The rope/scores chain ahead of attention values cut into slices: positions on both sides of the
-scores' 256-row chunks, the last row and past the capacity, head sizes of every vector layout, q, k and
-v from buffers and from a split linear's planes; the graph's results are those of the separate launches
-bit for bit, and those against a float64 reference."""
+"""The rope/scores chain and the softmax/values chain of attention values cut into slices: positions on
+both sides of the scores' 256-row chunks, the last row and past the capacity, head sizes of every vector
+layout, softmax rows of every width, q, k and v from buffers and from a split linear's planes; the
+graph's results are those of the separate launches bit for bit, and those against a float64 reference."""
 import numpy as np
 import pytest
 
@@ -24,7 +24,7 @@ def layer(x: _Rows, wq: Square, wk: Square, wv: Square, sincos: Rotary, position
 
 
 @pytest.mark.parametrize("b, a, t, d", [(1, 2, 1040, 128), (3, 1, 2100, 64), (1, 1, 6200, 20), (2, 2, 1500, 96), (1, 2, 600, 256),
-                                        (1, 9, 1030, 128)])
+                                        (1, 9, 1030, 128), (1, 1, 8192, 32), (2, 1, 512, 256)])
 def test_rope_scores(device, b, a, t, d):
     rng = np.random.default_rng(t + d)
     c = a * d
@@ -44,8 +44,9 @@ def test_rope_scores(device, b, a, t, d):
     bound = layer.lower(signature=types).compile(fuse_pointwise=False).bind(*buffers.values(), d ** -0.5)
     assert any(name.startswith("ckl_rope__rope__append_kv__attention_scores") and len(nodes) == 4
                for name, nodes in bound.units())
+    assert any(name.startswith("ckl_softmax__attention_values_split") and len(nodes) == 2 for name, nodes in bound.units())
     x = host["x"].astype(np.float64)
-    for p in (0, 1, 255, 256, 257, t - 1, t):
+    for p in (0, 1, 255, 256, 257, t // 2, t - 1, t):
         results = []
         for mode in ("ordinary", "graph", "graph", "stream"):
             for name in ("kc", "vc", "out"):
