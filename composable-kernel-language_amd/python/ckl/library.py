@@ -265,12 +265,12 @@ def _softmax(shapes, consts, ext):
 
 # Long contexts of few requests: a workgroup per (b, h) row leaves most of the chip idle, and one
 # workgroup streams only ~50 GB/s. The rows are then cut into slices (ckl_attention_values_split),
-# and the chain that needs a whole row in one workgroup is left for its parts (rope -> append_kv ->
-# scores, softmax, values): launches of about 6 us more (9 us for the figures here, rope -> append_kv
-# still apart), which at least 512 KB of values a row pay for, and
-# 16 KB more of them for every (b, h) row (attention layer, chain -> split, graph/ordinary us: 16 rows
-# of 8192 x 128 187/178 -> 61/83, of 1040 x 128 46/72 -> 43/66, of 512 x 128 31/60 -> 38/61; 64 rows of
-# 4096 x 128 113/134 -> 81/100, of 1040 x 128 49/75 -> 50/70; 128 rows of 2048 x 128 74/106 -> 80/101).
+# and the chain that needs a whole row in one workgroup becomes two launches (rope -> append_kv ->
+# scores, softmax -> values). At least 512 KB of values a row pay for that once about half the capacity
+# is in use, and 16 KB more of them for every (b, h) row (attention layer at the end of the capacity,
+# chain -> split, graph us: 16 rows of 8192 x 128 196 -> 66, of 1040 x 128 59 -> 52 (row 520 51 -> 50, row
+# 100 41 -> 47), of 700 x 128 46 -> 50 and of 512 x 128 43 -> 49 as three launches; 64 rows of 1040 x 128
+# 64 -> 59, but at row 520 53.5 -> 54.5; 128 rows of 2048 x 128 88 -> 90 as three launches).
 # About VALUES_SPLIT_GROUPS workgroups, but 16 slices or one per 128 KB (8 rows of 8192 x 64: 16 slices
 # 34.5, 64 37.4, 128 44.3 us: the last workgroup adds them; 4 rows of 8192 x 128: 16 41.0, 32 38.4).
 # One workgroup of 512 threads per compute unit (attention layer, us, 16 rows of 8192 x 128 / 64 rows of
